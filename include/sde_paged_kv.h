@@ -215,6 +215,15 @@ int sde_paged_attention(sde_kv_cache* cache, int layer, const float* d_q,
  * plan fits, and both entry points run the same plan. */
 #define SDE_NOALLOC_SCRATCH_BYTES ((size_t)4 << 20)
 
+/* Bytes of a second such array, for windows of many queries (a prompt or a
+ * chunk of one: at head sizes 64 / 128, 96 or more rows n_queries * nh/nkv
+ * per KV head and some 11 million rows x keys over all KV heads), whose
+ * kernel splits the context until one workgroup of 128 rows per CU is busy
+ * -- (CUs x 128 rows) x (dph + 2) x 4 bytes of partials, 17 MB on MI355X --
+ * whichever workspace it is given; where a captured call finds a smaller one
+ * in the cache, into fewer parts. */
+#define SDE_NOALLOC_WIDE_SCRATCH_BYTES ((size_t)18 << 20)
+
 /* sde_paged_attention without a workspace, allocating nothing: the
  * split-context partials go to a static device array of the library
  * (SDE_NOALLOC_SCRATCH_BYTES per device, held until the process ends) and

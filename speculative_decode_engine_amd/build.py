@@ -22,8 +22,8 @@ LIB_NAME = "libsde_paged.so"
 LIB_PATH = PKG_DIR / LIB_NAME
 OFFLOAD_ARCH = "gfx950"
 
-SOURCES = ["kv_cache.hip", "paged_attention.hip", "attention_generic.hip", "spec_accept.hip", "matvec.hip",
-           "model_loader.hip", "spec_loop.hip"]
+SOURCES = ["kv_cache.hip", "paged_attention.hip", "attention_window.hip",
+           "attention_generic.hip", "spec_accept.hip", "matvec.hip", "model_loader.hip", "spec_loop.hip"]
 
 # Measurement kernels for bench.py (a streaming read and the attention's
 # load skeleton): a library of their own, not part of the product.

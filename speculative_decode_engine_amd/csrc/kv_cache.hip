@@ -197,8 +197,20 @@ int finish_create(sde_kv_cache* c, sde_kv_cache** out) {
       hipMemset(c->d_counters, 0, (sde::kMaxAttnCounters + sde::kSpecScratchWords) *
                                       sizeof(uint32_t)) != hipSuccess ||
       hipDeviceGetAttribute(&c->n_cus, hipDeviceAttributeMultiprocessorCount, c->device) !=
-          hipSuccess ||
-      hipDeviceSynchronize() != hipSuccess) {
+          hipSuccess) {
+    release(c);
+    return SDE_ERR_HIP;
+  }
+  // The attention workspace ahead of the first call that needs one (contexts
+  // of more than one partition's 256 keys): a call that allocates waits for
+  // it, 20 us and more.  Larger plans still grow it.
+  if ((int64_t)cfg.max_blocks_per_layer * cfg.block_size > 256) {
+    if (hipMalloc(&c->workspace, sde::kInitialWorkspace) == hipSuccess)
+      c->workspace_bytes = sde::kInitialWorkspace;
+    else
+      (void)hipGetLastError();  // (left to the first call that needs it)
+  }
+  if (hipDeviceSynchronize() != hipSuccess) {
     release(c);
     return SDE_ERR_HIP;
   }

@@ -34,6 +34,7 @@
 
 #include "sde/attention_device.hpp"
 #include "attention_generic.hpp"
+#include "attention_window.hpp"
 #include "sde_internal.hpp"
 
 namespace sde {
@@ -176,6 +177,12 @@ size_t sde_grid_attention_workspace_size(int nh, int nkv, int dph, int n_queries
 
 namespace {
 
+// Whether a call without RoPE runs the wide-window kernel.
+bool serves_window(const sde_kv_cache* cache, int dph, int L_max, int nkv, int R) {
+  return !sde::gen::needs_generic(dph, cache->cfg.block_size) &&
+         sde::win::window_serves(L_max, nkv, R);
+}
+
 int run_attention(sde_kv_cache* cache, int layer, const float* d_q, float* d_out, int nh,
                   int nkv, int dph, int pos_base, int n_queries, void* d_workspace,
                   size_t workspace_bytes, sde_stream_t stream, const RopeArgs* rope,
@@ -189,6 +196,7 @@ int run_attention(sde_kv_cache* cache, int layer, const float* d_q, float* d_out
   const bool generic = sde::gen::needs_generic(dph, cache->cfg.block_size);
   StreamPlan plan{};
   sde::gen::GenPlan gplan{};
+  sde::win::WindowPlan wplan{};
   size_t need = 0;
   if (generic) {
     gplan = sde::gen::generic_plan(L_max, nkv, R, dph, cache->n_cus, parts_bound(L_max));
@@ -198,15 +206,36 @@ int run_attention(sde_kv_cache* cache, int layer, const float* d_q, float* d_out
     if ((int64_t)nkv * plan.row_groups > sde::kMaxAttnCounters) return SDE_ERR_UNSUPPORTED;
     need = partial_bytes(nkv, R, plan.n_parts, dph);
   }
+  const bool wide = !rope && serves_window(cache, dph, L_max, nkv, R);
+  if (wide) {
+    // A wide window: its own kernel and split.  Its partials take what the
+    // workspace holds (down to one partition, which needs none), and a call
+    // is refused for its workspace only where the 16-row kernels' plan is.
+    size_t most = SDE_NOALLOC_WIDE_SCRATCH_BYTES;
+    if (d_workspace) {
+      if (workspace_bytes < need) return SDE_ERR_WORKSPACE;
+      most = workspace_bytes < most ? workspace_bytes : most;
+    } else if (cache->workspace_used < most) {
+      hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+      if (hipStreamIsCapturing((hipStream_t)stream, &cap) != hipSuccess) return SDE_ERR_HIP;
+      if (cap != hipStreamCaptureStatusNone) {  // no allocation can be recorded
+        if (cache->workspace_used < need) return SDE_ERR_WORKSPACE;
+        most = cache->workspace_used;
+      }
+    }
+    wplan = sde::win::window_plan(L_max, nkv, R, dph, cache->n_cus, parts_bound(L_max), most);
+    need = sde::win::window_partial_bytes(wplan, nkv, R, dph);
+  }
   float* partials = nullptr;
   if (need > 0) {
     if (d_workspace) {
       if (workspace_bytes < need) return SDE_ERR_WORKSPACE;
       partials = static_cast<float*>(d_workspace);
     } else {
-      if (cache->workspace_bytes < need) {
-        // Grow the cache-owned workspace.  Not while the stream is being
-        // captured: the allocation cannot be recorded, and a graph would
+      if (cache->workspace_used < need) {
+        // Take more of the cache-owned workspace, growing it where what was
+        // allocated at creation does not do.  Not while the stream is being
+        // captured: an allocation cannot be recorded, and a graph would
         // keep its address.  The old buffer stays allocated (queued work
         // or an earlier graph may still use it) until the cache is freed,
         // so the size at least doubles: a context that grows call by call
@@ -214,12 +243,15 @@ int run_attention(sde_kv_cache* cache, int layer, const float* d_q, float* d_out
         hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
         if (hipStreamIsCapturing((hipStream_t)stream, &cap) != hipSuccess) return SDE_ERR_HIP;
         if (cap != hipStreamCaptureStatusNone) return SDE_ERR_WORKSPACE;
-        const size_t grow = need > 2 * cache->workspace_bytes ? need : 2 * cache->workspace_bytes;
-        void* grown = nullptr;
-        if (hipMalloc(&grown, grow) != hipSuccess) return SDE_ERR_HIP;
-        if (cache->workspace) cache->retired_workspaces.push_back(cache->workspace);
-        cache->workspace = grown;
-        cache->workspace_bytes = grow;
+        const size_t used = need > 2 * cache->workspace_used ? need : 2 * cache->workspace_used;
+        if (cache->workspace_bytes < used) {
+          void* grown = nullptr;
+          if (hipMalloc(&grown, used) != hipSuccess) return SDE_ERR_HIP;
+          if (cache->workspace) cache->retired_workspaces.push_back(cache->workspace);
+          cache->workspace = grown;
+          cache->workspace_bytes = used;
+        }
+        cache->workspace_used = used;
       }
       partials = static_cast<float*>(cache->workspace);
     }
@@ -250,6 +282,8 @@ int run_attention(sde_kv_cache* cache, int layer, const float* d_q, float* d_out
   a.n_parts = plan.n_parts;
   a.tiles_per_part = plan.tiles_per_part;
   a.qscale = (float)(kLog2e / std::sqrt((double)dph));
+  if (wide)
+    return sde::win::window_attention(a, wplan, dph, (hipStream_t)stream);
   // Each arrival counter on a 128-byte line of its own where they fit: a
   // split combine's waiting workgroups poll theirs while other groups'
   // arrivals update theirs.
@@ -366,21 +400,26 @@ constexpr int kMaxDevices = 64;
 // current device (scratch_address).  No part of it must start at zero
 // (each call writes every partial it later reads).
 static __device__ __align__(256) char scratch[SDE_NOALLOC_SCRATCH_BYTES];
+// The same for wide windows (sde::win), whose row groups are many more.
+static __device__ __align__(256) char wide_scratch[SDE_NOALLOC_WIDE_SCRATCH_BYTES];
 
 std::mutex g_scratch_mutex;
-std::atomic<void*> g_scratch_ptr[kMaxDevices];
+std::atomic<void*> g_scratch_ptr[2][kMaxDevices];
 
-// The device address of `scratch` on `device`, which must be current:
-// looked up on the first call on that device, then kept.
-int scratch_address(int device, void** out) {
+// The device address of `scratch` (or `wide_scratch`) on `device`, which
+// must be current: looked up on the first call on that device, then kept.
+int scratch_address(int device, bool wide, void** out) {
   if (device < 0 || device >= kMaxDevices) return SDE_ERR_UNSUPPORTED;
-  void* p = g_scratch_ptr[device].load(std::memory_order_acquire);
+  std::atomic<void*>& kept = g_scratch_ptr[wide ? 1 : 0][device];
+  void* p = kept.load(std::memory_order_acquire);
   if (!p) {
     std::lock_guard<std::mutex> lock(g_scratch_mutex);
-    p = g_scratch_ptr[device].load(std::memory_order_relaxed);
+    p = kept.load(std::memory_order_relaxed);
     if (!p) {
-      if (hipGetSymbolAddress(&p, HIP_SYMBOL(scratch)) != hipSuccess || !p) return SDE_ERR_HIP;
-      g_scratch_ptr[device].store(p, std::memory_order_release);
+      const hipError_t e = wide ? hipGetSymbolAddress(&p, HIP_SYMBOL(wide_scratch))
+                                : hipGetSymbolAddress(&p, HIP_SYMBOL(scratch));
+      if (e != hipSuccess || !p) return SDE_ERR_HIP;
+      kept.store(p, std::memory_order_release);
     }
   }
   *out = p;
@@ -397,10 +436,13 @@ extern "C" int sde_paged_attention_noalloc(sde_kv_cache* cache, int layer, const
   sde::DeviceGuard guard(cache->device);
   if (!guard.ok()) return SDE_ERR_HIP;
   void* ws = nullptr;
-  const int sst = scratch_address(cache->device, &ws);
+  const bool wide = serves_window(cache, dph, pos_base + n_queries, nkv,
+                                  n_queries * (nh / nkv));
+  const int sst = scratch_address(cache->device, wide, &ws);
   if (sst != SDE_OK) return sst;
   // A plan whose partials exceed the array gets SDE_ERR_WORKSPACE from
   // run_attention, before any launch; nothing here allocates.
   return run_attention(cache, layer, d_q, d_out, nh, nkv, dph, pos_base, n_queries, ws,
-                       SDE_NOALLOC_SCRATCH_BYTES, stream, nullptr);
+                       wide ? SDE_NOALLOC_WIDE_SCRATCH_BYTES : SDE_NOALLOC_SCRATCH_BYTES, stream,
+                       nullptr);
 }
