@@ -27,6 +27,12 @@ struct GenPlan {
 // more partials than SDE_NOALLOC_SCRATCH_BYTES holds.
 GenPlan generic_plan(int L_max, int nkv, int R, int dph, int n_cus, int max_parts);
 
+// Whether a shape runs the matrix-core form (gen_tile_kernel) of this path,
+// and its plan: row groups of 16, the partials within max_bytes.
+bool tile_serves(int dph, int block_size, int64_t pool_blocks);
+GenPlan tile_plan(int L_max, int nkv, int R, int dph, int n_cus, int max_parts,
+                  size_t max_bytes);
+
 // Bytes of partials the plan needs (0 for one partition).
 size_t generic_partial_bytes(const GenPlan& p, int nkv, int R, int dph);
 
@@ -37,7 +43,7 @@ size_t generic_partial_bytes(const GenPlan& p, int nkv, int R, int dph);
 int generic_attention(uint16_t* pool, const int32_t* table, int kv_dim, int block_size,
                       const float* q, float* out, float* partials, int nh, int nkv, int dph,
                       int pos_base, int n_queries, const GenPlan& plan,
-                      const GenRope* rope, hipStream_t stream);
+                      const GenRope* rope, uint32_t* counters, hipStream_t stream);
 
 }  // namespace gen
 }  // namespace sde

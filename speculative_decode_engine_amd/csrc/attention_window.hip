@@ -107,6 +107,13 @@ __device__ __forceinline__ void split_weights(const float (&x)[8], h8_t& hi, h8_
   }
 }
 
+// Weight of sums (max m, sum l) against the max `top`: 0 where no key was
+// seen; a sum of NaN logits alone (max -inf, sum NaN) is kept.
+__device__ __forceinline__ float sums_weight(float m, float l, float top) {
+  if (m == -INFINITY) return l == 0.f ? 0.f : 1.f;
+  return __builtin_amdgcn_exp2f(m - top);
+}
+
 __device__ __forceinline__ float half_max(float x) {
   const int v = __builtin_bit_cast(int, x);
   const auto h = __builtin_amdgcn_permlane32_swap(v, v, false, false);
@@ -516,8 +523,8 @@ __global__ __launch_bounds__(kWinThreads) void attn_window_kernel(AttnArgs a) {
   {
     const float2 y = *xml;
     const float m = fmaxf(m_row, y.x);
-    const float wa0 = m_row == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_row - m);
-    const float wa1 = y.x == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(y.x - m);
+    const float wa0 = sums_weight(m_row, l_row, m);
+    const float wa1 = sums_weight(y.x, y.y, m);
     m_row = m;
     l_row = l_row * wa0 + y.y * wa1;
 #pragma unroll
@@ -600,8 +607,7 @@ __global__ __launch_bounds__(256) void window_combine_kernel(AttnArgs a) {
     o.w *= old;
 #pragma unroll
     for (int i = 0; i < 4; i++) {
-      const float w =
-          p0 + i >= P || v[i].x == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(v[i].x - mx);
+      const float w = p0 + i >= P ? 0.f : sums_weight(v[i].x, v[i].y, mx);
       l += v[i].y * w;
       o.x += x[i].x * w;
       o.y += x[i].y * w;

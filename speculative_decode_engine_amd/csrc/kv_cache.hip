@@ -164,11 +164,9 @@ size_t pool_bytes_of(const sde_kv_config& c) {
 void release(sde_kv_cache* c) {
   if (!c) return;
   if (c->owns_pool && c->pool) (void)hipFree(c->pool);
-  if (c->d_tables) (void)hipFree(c->d_tables);
-  if (c->d_seq_len) (void)hipFree(c->d_seq_len);
-  if (c->workspace) (void)hipFree(c->workspace);
+  if (c->workspace && c->workspace != c->arena) (void)hipFree(c->workspace);
+  if (c->arena) (void)hipFree(c->arena);
   for (void* w : c->retired_workspaces) (void)hipFree(w);
-  if (c->d_counters) (void)hipFree(c->d_counters);
   delete c;
 }
 
@@ -187,28 +185,33 @@ int finish_create(sde_kv_cache* c, sde_kv_cache** out) {
       c->n_mapped[l] = cfg.max_blocks_per_layer;
     }
   }
-  if (hipMalloc(&c->d_tables, n_entries * sizeof(int32_t)) != hipSuccess ||
-      hipMemcpy(c->d_tables, c->h_tables.data(), n_entries * sizeof(int32_t),
+  // One allocation: the attention workspace (for caches of more than one
+  // partition's 256 keys: a call that has to allocate it takes 20 us and more
+  // longer; larger plans still grow it), the tables, the counters (zero at
+  // rest) and seq_len.
+  const size_t ws = (int64_t)cfg.max_blocks_per_layer * cfg.block_size > 256
+                        ? sde::kInitialWorkspace
+                        : 0;
+  const size_t tables = (n_entries * sizeof(int32_t) + 255) / 256 * 256;
+  const size_t counters =
+      ((size_t)sde::kMaxAttnCounters + sde::kSpecScratchWords) * sizeof(uint32_t);
+  if (hipMalloc(&c->arena, ws + tables + counters + sizeof(int32_t)) != hipSuccess) {
+    release(c);
+    return SDE_ERR_HIP;
+  }
+  char* base = static_cast<char*>(c->arena);
+  c->workspace = ws > 0 ? base : nullptr;
+  c->workspace_bytes = ws;
+  c->d_tables = reinterpret_cast<int32_t*>(base + ws);
+  c->d_counters = reinterpret_cast<uint32_t*>(base + ws + tables);
+  c->d_seq_len = reinterpret_cast<int32_t*>(base + ws + tables + counters);
+  if (hipMemcpy(c->d_tables, c->h_tables.data(), n_entries * sizeof(int32_t),
                 hipMemcpyHostToDevice) != hipSuccess ||
-      hipMalloc(&c->d_seq_len, sizeof(int32_t)) != hipSuccess ||
-      hipMemset(c->d_seq_len, 0, sizeof(int32_t)) != hipSuccess ||
-      hipMalloc(&c->d_counters, (sde::kMaxAttnCounters + sde::kSpecScratchWords) *
-                                    sizeof(uint32_t)) != hipSuccess ||
-      hipMemset(c->d_counters, 0, (sde::kMaxAttnCounters + sde::kSpecScratchWords) *
-                                      sizeof(uint32_t)) != hipSuccess ||
+      hipMemset(c->d_counters, 0, counters + sizeof(int32_t)) != hipSuccess ||
       hipDeviceGetAttribute(&c->n_cus, hipDeviceAttributeMultiprocessorCount, c->device) !=
           hipSuccess) {
     release(c);
     return SDE_ERR_HIP;
-  }
-  // The attention workspace ahead of the first call that needs one (contexts
-  // of more than one partition's 256 keys): a call that allocates waits for
-  // it, 20 us and more.  Larger plans still grow it.
-  if ((int64_t)cfg.max_blocks_per_layer * cfg.block_size > 256) {
-    if (hipMalloc(&c->workspace, sde::kInitialWorkspace) == hipSuccess)
-      c->workspace_bytes = sde::kInitialWorkspace;
-    else
-      (void)hipGetLastError();  // (left to the first call that needs it)
   }
   if (hipDeviceSynchronize() != hipSuccess) {
     release(c);

@@ -183,6 +183,26 @@ bool serves_window(const sde_kv_cache* cache, int dph, int L_max, int nkv, int R
          sde::win::window_serves(L_max, nkv, R);
 }
 
+// Lowers *most, the partials a plan may have, to what the call's workspace
+// holds: the caller's, or under stream capture (no allocation can be
+// recorded) what earlier calls took of the cache's.  SDE_ERR_WORKSPACE where
+// that is less than `need`.
+int workspace_limit(const sde_kv_cache* cache, size_t need, const void* d_workspace,
+                    size_t workspace_bytes, sde_stream_t stream, size_t* most) {
+  size_t have = *most;
+  if (d_workspace) {
+    have = workspace_bytes;
+  } else if (cache->workspace_used < *most) {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing((hipStream_t)stream, &cap) != hipSuccess) return SDE_ERR_HIP;
+    if (cap == hipStreamCaptureStatusNone) return SDE_OK;
+    have = cache->workspace_used;
+  }
+  if (have < need) return SDE_ERR_WORKSPACE;
+  if (have < *most) *most = have;
+  return SDE_OK;
+}
+
 int run_attention(sde_kv_cache* cache, int layer, const float* d_q, float* d_out, int nh,
                   int nkv, int dph, int pos_base, int n_queries, void* d_workspace,
                   size_t workspace_bytes, sde_stream_t stream, const RopeArgs* rope,
@@ -198,9 +218,21 @@ int run_attention(sde_kv_cache* cache, int layer, const float* d_q, float* d_out
   sde::gen::GenPlan gplan{};
   sde::win::WindowPlan wplan{};
   size_t need = 0;
+  bool tiles = false;
   if (generic) {
     gplan = sde::gen::generic_plan(L_max, nkv, R, dph, cache->n_cus, parts_bound(L_max));
     need = sde::gen::generic_partial_bytes(gplan, nkv, R, dph);
+    tiles = sde::gen::tile_serves(dph, cache->cfg.block_size, cache->cfg.pool_blocks);
+    if (tiles) {
+      // The matrix-core form has a plan of its own; its partials take what
+      // the workspace holds, and a call is refused for its workspace only
+      // where the fp32 form's plan is.
+      size_t most = SDE_NOALLOC_SCRATCH_BYTES;
+      const int st = workspace_limit(cache, need, d_workspace, workspace_bytes, stream, &most);
+      if (st != SDE_OK) return st;
+      gplan = sde::gen::tile_plan(L_max, nkv, R, dph, cache->n_cus, parts_bound(L_max), most);
+      need = sde::gen::generic_partial_bytes(gplan, nkv, R, dph);
+    }
   } else {
     plan = plan_for(L_max, nkv, R, cache->n_cus);
     if ((int64_t)nkv * plan.row_groups > sde::kMaxAttnCounters) return SDE_ERR_UNSUPPORTED;
@@ -212,17 +244,8 @@ int run_attention(sde_kv_cache* cache, int layer, const float* d_q, float* d_out
     // workspace holds (down to one partition, which needs none), and a call
     // is refused for its workspace only where the 16-row kernels' plan is.
     size_t most = SDE_NOALLOC_WIDE_SCRATCH_BYTES;
-    if (d_workspace) {
-      if (workspace_bytes < need) return SDE_ERR_WORKSPACE;
-      most = workspace_bytes < most ? workspace_bytes : most;
-    } else if (cache->workspace_used < most) {
-      hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-      if (hipStreamIsCapturing((hipStream_t)stream, &cap) != hipSuccess) return SDE_ERR_HIP;
-      if (cap != hipStreamCaptureStatusNone) {  // no allocation can be recorded
-        if (cache->workspace_used < need) return SDE_ERR_WORKSPACE;
-        most = cache->workspace_used;
-      }
-    }
+    const int st = workspace_limit(cache, need, d_workspace, workspace_bytes, stream, &most);
+    if (st != SDE_OK) return st;
     wplan = sde::win::window_plan(L_max, nkv, R, dph, cache->n_cus, parts_bound(L_max), most);
     need = sde::win::window_partial_bytes(wplan, nkv, R, dph);
   }
@@ -247,7 +270,8 @@ int run_attention(sde_kv_cache* cache, int layer, const float* d_q, float* d_out
         if (cache->workspace_bytes < used) {
           void* grown = nullptr;
           if (hipMalloc(&grown, used) != hipSuccess) return SDE_ERR_HIP;
-          if (cache->workspace) cache->retired_workspaces.push_back(cache->workspace);
+          if (cache->workspace && cache->workspace != cache->arena)
+            cache->retired_workspaces.push_back(cache->workspace);
           cache->workspace = grown;
           cache->workspace_bytes = used;
         }
@@ -261,6 +285,7 @@ int run_attention(sde_kv_cache* cache, int layer, const float* d_q, float* d_out
     return sde::gen::generic_attention(cache->pool, sde::layer_table(cache, layer),
                                        cache->cfg.kv_dim, cache->cfg.block_size, d_q, d_out,
                                        partials, nh, nkv, dph, pos_base, n_queries, gplan, grope,
+                                       tiles ? cache->d_counters : nullptr,
                                        (hipStream_t)stream);
 
   AttnArgs a;

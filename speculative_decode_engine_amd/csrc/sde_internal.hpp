@@ -19,6 +19,7 @@ struct sde_kv_cache {
   uint16_t* pool = nullptr;
   size_t pool_bytes = 0;
   bool owns_pool = false;
+  void* arena = nullptr;                // workspace, tables, counters, seq_len
   int32_t* d_tables = nullptr;          // [n_layers][max_blocks_per_layer]
   std::vector<int32_t> h_tables;        // host mirror of d_tables
   std::vector<int32_t> n_mapped;        // leading mapped logical blocks per layer

@@ -1,0 +1,95 @@
+"""GPU parity of the matrix-core form of the generic attention path (head
+sizes that are multiples of 8 up to 256, any block size: gen_tile_kernel)
+against the fp64 oracle.
+
+A workgroup there takes 16 rows -- (query, head in group) pairs of a KV head
+-- and its four waves 32-token tiles in turn; a tile is loaded as a flat run
+of 16-byte units, so the head size in units (odd, even, a multiple of 4, 8,
+16) decides the lanes' tokens, the LDS swizzle and the tail load, and the
+head size within its padding to 32 what must be dropped.  The shapes go over
+those, over row groups that are not full, one row past a group, contexts that
+end inside a tile or fill partitions exactly, none at all, and block sizes
+that no tile aligns with.
+
+Tolerance: products carry ~22 bits of q and the weights, sums are fp32: some
+1e-6 of the output's scale; the bound is 1e-5 of it."""
+import numpy as np
+import pytest
+import torch
+
+from conftest import case_banner
+from speculative_decode_engine_amd import workloads as W
+from test_gpu_attention import assert_close, build_layer
+
+pytestmark = pytest.mark.gpu
+
+
+def check(got, ref, what):
+    assert_close(got, ref, what)
+    scale = np.abs(ref).max()
+    err = np.abs(got.astype(np.float64) - ref).max()
+    assert err <= 1e-5 * scale, f"{what}: max abs err {err:.3e}, output scale {scale:.3e}"
+
+
+SIZES = [(4, 2, dph, bs, ctx, 3)
+         for dph, bs, ctx in [(8, 16, 130), (16, 8, 255), (24, 5, 300), (32, 16, 1000),
+                              (40, 16, 511), (48, 1, 77), (56, 32, 640), (72, 16, 1023),
+                              (80, 7, 900), (88, 16, 129), (96, 24, 2045), (104, 16, 64),
+                              (112, 16, 1500), (120, 48, 95), (136, 16, 700), (160, 9, 515),
+                              (168, 16, 31), (184, 16, 1280), (192, 64, 257), (200, 16, 900),
+                              (232, 3, 700), (248, 16, 385), (256, 16, 3000), (64, 12, 1000),
+                              (128, 20, 1000)]]
+ROWS = [
+    (16, 1, 96, 16, 500, 1),     # 16 rows: one full group
+    (17, 1, 96, 16, 500, 1),     # one row past it
+    (5, 5, 80, 16, 5000, 1),     # one row per KV head, many partitions
+    (6, 2, 256, 16, 0, 50),      # 150 rows, no context: groups that see little of the window
+    (32, 32, 96, 16, 4095, 1),   # a context that fills its last tile
+    (7, 1, 112, 16, 16300, 9),   # 63 rows, long context
+    (8, 8, 32, 16, 127, 1),      # one partition exactly
+    (8, 8, 32, 16, 128, 1),      # and one key more
+    (2, 2, 224, 16, 0, 1),       # the window's own key alone
+]
+
+
+@pytest.mark.parametrize("nh,nkv,dph,bs,ctx,M", SIZES + ROWS)
+def test_tile_form_matches_float64(gpu, oracle, nh, nkv, dph, bs, ctx, M):
+    case_banner("tile form", nh, nkv, dph, bs, ctx, M)
+    cache, K, V, rng = build_layer(nh, nkv, dph, bs, ctx, M, -(-(ctx + M) // bs) + 9, dph + ctx)
+    q = W.queries(rng, M, nh, dph)
+    qt = torch.from_numpy(q).cuda()
+    nan = torch.full((M, nh * dph), float("nan"), device="cuda")
+    out = cache.attention(0, qt, nh, nkv, dph, ctx, out=nan.clone())
+    again = cache.attention_noalloc(0, qt, nh, nkv, dph, ctx, out=nan.clone())
+    ws = torch.empty(max(4, cache.workspace_size(nh, nkv, dph, M, ctx + M)) // 4, device="cuda")
+    third = cache.attention(0, qt, nh, nkv, dph, ctx, out=nan.clone(), workspace=ws)
+    torch.cuda.synchronize()
+    assert torch.equal(out, again) and torch.equal(out, third)
+    ref = oracle.attention_f64_np(q, K, V, nh, nkv, dph, ctx)
+    check(out.cpu().numpy(), ref, f"dph {dph} bs {bs} ctx {ctx}")
+    cache.free()
+
+
+@pytest.mark.parametrize("dph,bs", [(24, 16), (96, 16), (256, 7)])
+def test_tile_form_hidden_nonfinite_rows(gpu, oracle, dph, bs):
+    """Inf / NaN in V and NaN in K at a window position, and stale NaN past
+    the window, reach only the queries that see them; fp16 padding features
+    never reach an output."""
+    case_banner("tile form, hidden non-finite", dph, bs)
+    nh, nkv, ctx, M = 4, 2, 200, 9
+    cache, K, V, rng = build_layer(nh, nkv, dph, bs, ctx, M, 60, dph)
+    bad = ctx + 4
+    k, v = K[bad].copy(), V[bad].copy()
+    v[::3], v[1::3], k[5] = np.inf, np.nan, np.nan
+    cache.append(0, torch.from_numpy(k[None]).cuda(), torch.from_numpy(v[None]).cuda(), bad)
+    last = ctx + M
+    if last % bs:
+        table = cache.block_table(0)
+        cache.pool_blocks_view()[int(table[last // bs]), :, last % bs:] = 0x7E00  # NaN
+    q = W.queries(rng, M, nh, dph)
+    out = cache.attention(0, torch.from_numpy(q).cuda(), nh, nkv, dph, ctx).cpu().numpy()
+    ref = oracle.attention_f64_np(q[:4], K[:bad], V[:bad], nh, nkv, dph, ctx)
+    check(out[:4], ref, "queries that do not see it")
+    # (KV head 0's rows hold the NaN key: not finite from query 4 on)
+    assert not np.isfinite(out[4:, :dph]).any()
+    cache.free()
