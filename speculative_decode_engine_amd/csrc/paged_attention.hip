@@ -30,6 +30,7 @@
 #include <climits>
 #include <cmath>
 #include <cstdlib>
+#include <cstring>
 #include <mutex>
 
 #include "sde/attention_device.hpp"
@@ -319,6 +320,27 @@ int run_attention(sde_kv_cache* cache, int layer, const float* d_q, float* d_out
   return dph == 128 ? launch<128>(plan, a, nkv, s, rope) : launch<64>(plan, a, nkv, s, rope);
 }
 
+// theta^(-2j/dph) for j < dph / 2 (then zeros to kMaxDph / 2), computed in
+// double precision and rounded to fp32.  Every layer of a model asks for the
+// same ones: a thread keeps the last it formed (64 exponentials, 1 us of a
+// call's host time).
+const float* rope_frequencies(double theta, int dph) {
+  struct Table {
+    double theta = 0.0;
+    int dph = 0;
+    float inv[sde::gen::kMaxDph / 2];
+  };
+  thread_local Table t;
+  if (t.dph != dph || t.theta != theta) {
+    const double log_theta = std::log(theta);
+    for (int j = 0; j < sde::gen::kMaxDph / 2; j++)
+      t.inv[j] = j < dph / 2 ? (float)std::exp(-log_theta * (2.0 * j) / dph) : 0.f;
+    t.theta = theta;
+    t.dph = dph;
+  }
+  return t.inv;
+}
+
 }  // namespace
 
 extern "C" {
@@ -361,7 +383,7 @@ int sde_rope_append_attention(sde_kv_cache* cache, int layer, const float* d_q,
   const bool div = (rope->scaling_type == SDE_ROPE_LINEAR || rope->scaling_type == SDE_ROPE_YARN) &&
                    factor > 1.0;
   rp.pos_div = div ? rope->scaling_factor : 1.0f;
-  const double log_theta = std::log(theta);
+  const float* inv_freq = rope_frequencies(theta, dph);
   if (sde::gen::needs_generic(dph, cache->cfg.block_size)) {
     // the generic path: RoPE of k and the append, then attention with q
     // rotated in-kernel (same frequency rule, up to dph / 2 = 256 pairs)
@@ -369,13 +391,11 @@ int sde_rope_append_attention(sde_kv_cache* cache, int layer, const float* d_q,
     gr.k_new = d_k;
     gr.v_new = d_v;
     gr.pos_div = rp.pos_div;
-    for (int j = 0; j < sde::gen::kMaxDph / 2; j++)
-      gr.inv_freq[j] = j < dph / 2 ? (float)std::exp(-log_theta * (2.0 * j) / dph) : 0.f;
+    std::memcpy(gr.inv_freq, inv_freq, sizeof(gr.inv_freq));
     return run_attention(cache, layer, d_q, d_out, nh, nkv, dph, pos_base, n_queries,
                          d_workspace, workspace_bytes, stream, nullptr, &gr);
   }
-  for (int j = 0; j < 64; j++)
-    rp.inv_freq[j] = j < dph / 2 ? (float)std::exp(-log_theta * (2.0 * j) / dph) : 0.f;
+  std::memcpy(rp.inv_freq, inv_freq, sizeof(rp.inv_freq));
   return run_attention(cache, layer, d_q, d_out, nh, nkv, dph, pos_base, n_queries,
                        d_workspace, workspace_bytes, stream, &rp);
 }

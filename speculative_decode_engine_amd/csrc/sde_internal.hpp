@@ -60,10 +60,13 @@ class DeviceGuard {
  public:
   explicit DeviceGuard(int dev) {
     if (hipGetDevice(&prev_) != hipSuccess) prev_ = -1;
-    if (prev_ != dev) ok_ = hipSetDevice(dev) == hipSuccess;
+    if (prev_ != dev) {
+      ok_ = hipSetDevice(dev) == hipSuccess;
+      changed_ = true;
+    }
   }
   ~DeviceGuard() {
-    if (prev_ >= 0 && ok_) (void)hipSetDevice(prev_);
+    if (changed_ && prev_ >= 0 && ok_) (void)hipSetDevice(prev_);
   }
   bool ok() const { return ok_; }
   DeviceGuard(const DeviceGuard&) = delete;
@@ -72,6 +75,7 @@ class DeviceGuard {
  private:
   int prev_ = -1;
   bool ok_ = true;
+  bool changed_ = false;
 };
 
 // Tokens [0, mapped_tokens) of a layer have a physical block.

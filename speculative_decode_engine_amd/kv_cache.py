@@ -62,6 +62,29 @@ def _stream_handle(stream: Optional[torch.cuda.Stream]) -> ctypes.c_void_p:
     return ctypes.c_void_p(s.cuda_stream)
 
 
+# The current stream's handle without a Stream object for each call (1 us of a
+# call's 4); where this torch lacks the raw accessors, the public way.
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+_raw_device = getattr(torch._C, "_cuda_getDevice", None)
+
+
+def _stream(stream: Optional[torch.cuda.Stream]) -> int:
+    if stream is None and _raw_stream is not None and _raw_device is not None:
+        return _raw_stream(_raw_device())
+    return _stream_handle(stream).value or 0
+
+
+_F32 = torch.float32
+
+
+def _is_f32(t, shape: tuple) -> bool:
+    """Whether t is what _dev_f32 returns unchanged: a plain contiguous CUDA
+    float32 tensor of this shape (a call's usual case, told in one pass; any
+    other goes through _dev_f32, which says what is wrong with it)."""
+    return (type(t) is torch.Tensor and t.is_cuda and t.dtype is _F32 and t.shape == shape
+            and t.is_contiguous())
+
+
 def _dev_f32(t: torch.Tensor, name: str, shape: tuple) -> torch.Tensor:
     if not isinstance(t, torch.Tensor) or t.device.type != "cuda":
         raise TypeError(f"{name} must be a CUDA tensor")
@@ -144,6 +167,15 @@ class KVCache:
             raise RuntimeError("cache has been freed")
         return self._handle
 
+    def _rows(self, t: torch.Tensor, name: str, m: int, width: int) -> torch.Tensor:
+        shape = (m, width)
+        return t if _is_f32(t, shape) else _dev_f32(t.reshape(m, width), name, shape)
+
+    def _out(self, out: Optional[torch.Tensor], m: int, width: int) -> torch.Tensor:
+        if out is None:
+            return torch.empty(m, width, dtype=_F32, device=self.device)
+        return out if _is_f32(out, (m, width)) else _dev_f32(out, "out", (m, width))
+
     # ---- metadata -------------------------------------------------------------
     def pool_blocks_view(self) -> torch.Tensor:
         """The pool as int16 [pool_blocks][2][block_size][kv_dim] (torch pools)."""
@@ -179,16 +211,16 @@ class KVCache:
 
     def set_seq_len(self, n: int, stream=None) -> None:
         """set_seq_len_kernel (kernels.cu:546-548)."""
-        check(self._lib.sde_kv_set_seq_len(self.handle, n, _stream_handle(stream)),
+        check(self._lib.sde_kv_set_seq_len(self.handle, n, _stream(stream)),
               "set_seq_len")
 
     def reset(self, stream=None) -> None:
         """kv_cache_reset (kv_cache.cu:50-52)."""
-        check(self._lib.sde_kv_reset(self.handle, _stream_handle(stream)), "kv_cache_reset")
+        check(self._lib.sde_kv_reset(self.handle, _stream(stream)), "kv_cache_reset")
 
     def rollback(self, target_len: int, stream=None) -> None:
         """O(1) rewind of rejected drafts (kernels.cu:2457-2459): no pool bytes move."""
-        check(self._lib.sde_kv_rollback(self.handle, target_len, _stream_handle(stream)),
+        check(self._lib.sde_kv_rollback(self.handle, target_len, _stream(stream)),
               "kv_cache_rollback")
 
     def device_seq_len(self) -> int:
@@ -203,11 +235,10 @@ class KVCache:
         """cublas_kv_append_kernel (kernels.cu:826-844): fp32 [M][kv_dim] rows
         -> fp16 (RNE) at positions pos_base..pos_base+M-1."""
         M = k.shape[0] if k.dim() == 2 else 1
-        k = _dev_f32(k.reshape(M, self.kv_dim), "k", (M, self.kv_dim))
-        v = _dev_f32(v.reshape(M, self.kv_dim), "v", (M, self.kv_dim))
-        check(self._lib.sde_kv_append(self.handle, layer, ctypes.c_void_p(k.data_ptr()),
-                                      ctypes.c_void_p(v.data_ptr()), pos_base, M,
-                                      _stream_handle(stream)), "kv_cache_append")
+        k = self._rows(k, "k", M, self.kv_dim)
+        v = self._rows(v, "v", M, self.kv_dim)
+        check(self._lib.sde_kv_append(self.handle, layer, k.data_ptr(), v.data_ptr(), pos_base,
+                                      M, _stream(stream)), "kv_cache_append")
 
     def write_fp16(self, layer: int, k16: torch.Tensor, v16: torch.Tensor, pos_base: int,
                    stream=None) -> None:
@@ -244,20 +275,16 @@ class KVCache:
         device_attention_dispatch (attention.h:140-164): q fp32 [M][nh*dph];
         query m attends causally to positions [0, pos_base+m]."""
         M = q.shape[0] if q.dim() == 2 else 1
-        q = _dev_f32(q.reshape(M, nh * dph), "q", (M, nh * dph))
-        if out is None:
-            out = torch.empty(M, nh * dph, dtype=torch.float32, device=self.device)
-        _dev_f32(out, "out", (M, nh * dph))
+        q = self._rows(q, "q", M, nh * dph)
+        out = self._out(out, M, nh * dph)
         ws_ptr, ws_bytes = None, 0
         if workspace is not None:
             if workspace.device.type != "cuda" or not workspace.is_contiguous():
                 raise ValueError("workspace must be a contiguous CUDA tensor")
             ws_ptr, ws_bytes = workspace.data_ptr(), workspace.numel() * workspace.element_size()
         check(self._lib.sde_attention_dispatch(
-            attn_type, self.handle, layer, ctypes.c_void_p(q.data_ptr()),
-            ctypes.c_void_p(out.data_ptr()), nh, nkv, dph, pos_base, M,
-            ctypes.c_void_p(ws_ptr), ws_bytes, _stream_handle(stream)),
-            "paged_attention")
+            attn_type, self.handle, layer, q.data_ptr(), out.data_ptr(), nh, nkv, dph, pos_base, M,
+            ws_ptr, ws_bytes, _stream(stream)), "paged_attention")
         return out
 
     def attention_noalloc(self, layer: int, q: torch.Tensor, nh: int, nkv: int, dph: int,
@@ -267,13 +294,11 @@ class KVCache:
         to the library's static per-device array, so the call allocates no
         device memory (out must then be given by the caller)."""
         M = q.shape[0] if q.dim() == 2 else 1
-        q = _dev_f32(q.reshape(M, nh * dph), "q", (M, nh * dph))
-        if out is None:
-            out = torch.empty(M, nh * dph, dtype=torch.float32, device=self.device)
-        _dev_f32(out, "out", (M, nh * dph))
+        q = self._rows(q, "q", M, nh * dph)
+        out = self._out(out, M, nh * dph)
         check(self._lib.sde_paged_attention_noalloc(
-            self.handle, layer, ctypes.c_void_p(q.data_ptr()), ctypes.c_void_p(out.data_ptr()),
-            nh, nkv, dph, pos_base, M, _stream_handle(stream)), "paged_attention_noalloc")
+            self.handle, layer, q.data_ptr(), out.data_ptr(), nh, nkv, dph, pos_base, M,
+            _stream(stream)), "paged_attention_noalloc")
         return out
 
     def rope_append_attention(self, layer: int, q: torch.Tensor, k: torch.Tensor,
@@ -289,12 +314,10 @@ class KVCache:
         model.cu:281-323) at positions pos_base+m, k and v appended there,
         and query m attends causally to [0, pos_base+m]."""
         M = q.shape[0] if q.dim() == 2 else 1
-        q = _dev_f32(q.reshape(M, nh * dph), "q", (M, nh * dph))
-        k = _dev_f32(k.reshape(M, self.kv_dim), "k", (M, self.kv_dim))
-        v = _dev_f32(v.reshape(M, self.kv_dim), "v", (M, self.kv_dim))
-        if out is None:
-            out = torch.empty(M, nh * dph, dtype=torch.float32, device=self.device)
-        _dev_f32(out, "out", (M, nh * dph))
+        q = self._rows(q, "q", M, nh * dph)
+        k = self._rows(k, "k", M, self.kv_dim)
+        v = self._rows(v, "v", M, self.kv_dim)
+        out = self._out(out, M, nh * dph)
         ws_ptr, ws_bytes = None, 0
         if workspace is not None:
             if workspace.device.type != "cuda" or not workspace.is_contiguous():
@@ -302,10 +325,9 @@ class KVCache:
             ws_ptr, ws_bytes = workspace.data_ptr(), workspace.numel() * workspace.element_size()
         rope = _native.RopeConfig(theta, scaling_type, scaling_factor)
         check(self._lib.sde_rope_append_attention(
-            self.handle, layer, ctypes.c_void_p(q.data_ptr()), ctypes.c_void_p(k.data_ptr()),
-            ctypes.c_void_p(v.data_ptr()), ctypes.c_void_p(out.data_ptr()), nh, nkv, dph,
-            pos_base, M, ctypes.byref(rope), ctypes.c_void_p(ws_ptr), ws_bytes,
-            _stream_handle(stream)), "rope_append_attention")
+            self.handle, layer, q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), nh, nkv,
+            dph, pos_base, M, ctypes.byref(rope), ws_ptr, ws_bytes, _stream(stream)),
+            "rope_append_attention")
         return out
 
 

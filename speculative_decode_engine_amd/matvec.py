@@ -12,7 +12,25 @@ import torch
 
 from . import _native
 from ._native import check
-from .kv_cache import _stream_handle
+from .kv_cache import _F32, _stream, _stream_handle
+
+
+def _rows_f32(x) -> bool:
+    """A call's usual operand, told in one pass."""
+    return type(x) is torch.Tensor and x.is_cuda and x.dtype is _F32 and x.is_contiguous()
+
+
+def _check_x(x2) -> None:
+    if not _rows_f32(x2) and (x2.device.type != "cuda" or x2.dtype != torch.float32
+                              or not x2.is_contiguous()):
+        raise TypeError("x must be a contiguous CUDA float32 tensor")
+
+
+def _check_out(out, m: int, d_out: int) -> None:
+    if out.numel() != m * d_out or not _rows_f32(out) and (
+            out.device.type != "cuda" or out.dtype != torch.float32 or not out.is_contiguous()):
+        raise TypeError(f"out must be a contiguous CUDA float32 tensor of {m}x{d_out}")
+
 
 _WORKSPACES: dict = {}
 _RETIRED: list = []
@@ -35,7 +53,7 @@ def _cached_workspace(d_in: int, d_out: int, n_rows: int, device, stream) -> tor
     or a captured graph may still use it)."""
     lib = _native.load()
     need = int(lib.sde_matvec_workspace_size(d_in, d_out, n_rows))
-    key = (torch.device(device), _stream_handle(stream).value or 0)
+    key = (torch.device(device), _stream(stream))
     ws = _WORKSPACES.get(key)
     if ws is None or ws.numel() < need:
         if ws is not None:
@@ -56,8 +74,7 @@ def matvec(x: torch.Tensor, W: torch.Tensor, out: Optional[torch.Tensor] = None,
     workspace defaults to one cached per (device, stream)."""
     squeeze = x.dim() == 1
     x2 = x.unsqueeze(0) if squeeze else x
-    if x2.device.type != "cuda" or x2.dtype != torch.float32 or not x2.is_contiguous():
-        raise TypeError("x must be a contiguous CUDA float32 tensor")
+    _check_x(x2)
     if W.device.type != "cuda" or W.dtype != torch.float16 or not W.is_contiguous() or W.dim() != 2:
         raise TypeError("W must be a contiguous 2-D CUDA float16 tensor")
     M, d_in = x2.shape
@@ -67,18 +84,15 @@ def matvec(x: torch.Tensor, W: torch.Tensor, out: Optional[torch.Tensor] = None,
     if out is None:
         if accumulate:
             raise ValueError("accumulate needs out")
-        out = torch.empty((M, d_out) if not squeeze else (d_out,), dtype=torch.float32,
-                          device=x.device)
-    if out.device.type != "cuda" or out.dtype != torch.float32 or not out.is_contiguous() \
-            or out.numel() != M * d_out:
-        raise TypeError(f"out must be a contiguous CUDA float32 tensor of {M}x{d_out}")
+        out = torch.empty((M, d_out) if not squeeze else (d_out,), dtype=_F32, device=x.device)
+    else:
+        _check_out(out, M, d_out)
     if workspace is None:
         workspace = _cached_workspace(d_in, d_out, M, x.device, stream)
     lib = _native.load()
-    check(lib.sde_matvec(ctypes.c_void_p(x2.data_ptr()), ctypes.c_void_p(W.data_ptr()),
-                         ctypes.c_void_p(out.data_ptr()), d_in, d_out, M, int(bool(accumulate)),
-                         ctypes.c_void_p(workspace.data_ptr()), workspace.numel(),
-                         _stream_handle(stream)), "matvec")
+    check(lib.sde_matvec(x2.data_ptr(), W.data_ptr(), out.data_ptr(), d_in, d_out, M,
+                         int(bool(accumulate)), workspace.data_ptr(), workspace.numel(),
+                         _stream(stream)), "matvec")
     return out
 
 
@@ -108,21 +122,18 @@ def matvec_packed(x: torch.Tensor, Wp: PackedWeight, out: Optional[torch.Tensor]
     sum_r x[m][r] * W[r][c], x CUDA float32 [M][d_in] or [d_in] (M <= 16)."""
     squeeze = x.dim() == 1
     x2 = x.unsqueeze(0) if squeeze else x
-    if x2.device.type != "cuda" or x2.dtype != torch.float32 or not x2.is_contiguous():
-        raise TypeError("x must be a contiguous CUDA float32 tensor")
+    _check_x(x2)
     M, d_in = x2.shape
     if d_in != Wp.d_in:
         raise ValueError(f"W has {Wp.d_in} rows, x has {d_in} columns")
     if out is None:
         if accumulate:
             raise ValueError("accumulate needs out")
-        out = torch.empty((M, Wp.d_out) if not squeeze else (Wp.d_out,), dtype=torch.float32,
+        out = torch.empty((M, Wp.d_out) if not squeeze else (Wp.d_out,), dtype=_F32,
                           device=x.device)
-    if out.device.type != "cuda" or out.dtype != torch.float32 or not out.is_contiguous() \
-            or out.numel() != M * Wp.d_out:
-        raise TypeError(f"out must be a contiguous CUDA float32 tensor of {M}x{Wp.d_out}")
-    lib = _native.load()
-    check(lib.sde_matvec_packed(ctypes.c_void_p(x2.data_ptr()), ctypes.c_void_p(Wp.data.data_ptr()),
-                                ctypes.c_void_p(out.data_ptr()), d_in, Wp.d_out, M,
-                                int(bool(accumulate)), _stream_handle(stream)), "matvec_packed")
+    else:
+        _check_out(out, M, Wp.d_out)
+    check(_native.load().sde_matvec_packed(x2.data_ptr(), Wp.data.data_ptr(), out.data_ptr(), d_in,
+                                           Wp.d_out, M, int(bool(accumulate)), _stream(stream)),
+          "matvec_packed")
     return out
