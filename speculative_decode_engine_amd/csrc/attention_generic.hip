@@ -52,14 +52,11 @@ __global__ __launch_bounds__(kThreads) void gen_rope_append_kernel(GenArgs a, Ge
 //  * logits K . Q^T and output V^T . P^T are 16x16x32 fp16 MFMA over the
 //    head size padded to 32, q and the weights as fp16 hi + lo pairs, sums
 //    in fp32 (the layouts of attention_device.hpp's tile path);
-//  * the waves' sums meet in LDS, the partitions' in a combine run by the
-//    last workgroup of a (KV head, row group) to finish (a kernel of its own,
-//    a thread per feature walking the partitions one load after another, took
-//    13-15 us).
+//  * the waves' sums meet in LDS, the partitions' in a combine kernel.
 // Bound by the latency of a few tiles in turn and, as they grow, by memory.
 // Measured on MI355X, us per layer, fp32 form / this: decode over 3000 keys,
-// 32 KV heads of 96, 188 + 13 (combine) / 17.4; a 5-query window over 4000
-// keys, 16/8 heads of 256, RoPE of q included, 193 + 15 / 32.4.  Errors
+// 32 KV heads of 96, 188 + 13 (combine) / 17.3 in all; a 5-query window over
+// 4000 keys, 16/8 heads of 256, RoPE of q included, 193 + 15 / 28.  Errors
 // against float64 fell too (4.7e-7 -> 3.0e-7, 6.5e-7 -> 4.2e-7 of the
 // output's norm): shorter sums.
 // DPHP: the head size rounded up to a multiple of 32.
@@ -78,6 +75,8 @@ struct TileShape {
   static constexpr int NI = DPHP / 16;                     // wave loads of a tile (at most)
   static constexpr int TILEB = attn::kTile * 2 * DPHP;     // a staged tile (at most)
   static constexpr int WAVEB = 2 * TILEB;                  // a wave's K and V tile
+  // the next smaller form's head size: features below it always exist
+  static constexpr int kLeast = DPHP == 256 ? 192 : DPHP - 32;
 };
 
 template <int DPHP>
@@ -88,8 +87,6 @@ struct TileLds {
   char st[kTileWaves * Sh::WAVEB + 1024] __attribute__((aligned(16)));
   h8_t qop[2 * Sh::KS * 64];
   float2 ml[kTileWaves][kTileRows];
-  float wgt[kTileRows][attn::kStreamMaxParts + 1];  // a row's partition weights, then 1 / sum
-  int last;
   static_assert(kTileRows * DPHP * 4 <= Sh::WAVEB, "a wave's sums fit its tiles");
 };
 
@@ -125,8 +122,7 @@ __device__ __forceinline__ float part_weight(float2 ml, float mx) {
 
 template <int DPHP>
 __global__ __launch_bounds__(64 * kTileWaves) void gen_tile_kernel(GenArgs a, GenRope rp,
-                                                                   int use_rope,
-                                                                   uint32_t* counters) {
+                                                                   int use_rope) {
   using Sh = TileShape<DPHP>;
   __shared__ TileLds<DPHP> lds;
   constexpr float kNegInf = -__builtin_inff();
@@ -157,14 +153,15 @@ __global__ __launch_bounds__(64 * kTileWaves) void gen_tile_kernel(GenArgs a, Ge
   const int ni = (U + 1) / 2;  // 32 U units, 64 per load
   const size_t row_bytes = 2 * (size_t)a.kv_dim;
   const char* head = reinterpret_cast<const char*>(a.pool) + (size_t)kvh * dph * 2;
-  // lane l's token of load j and the byte offset of its unit in the row
-  int tok[Sh::NI], uoff[Sh::NI];
+  // lane l's token of load j (low 5 bits) and the byte offset of its unit in
+  // the row (a multiple of 16)
+  int at[Sh::NI];
 #pragma unroll
   for (int j = 0; j < Sh::NI; j++) {
     const int f = 64 * j + lane;
-    tok[j] = min(f / U, attn::kTile - 1);
+    const int t = min(f / U, attn::kTile - 1);
     const int u = f - (f / U) * U;
-    uoff[j] = 16 * (u ^ ((tok[j] >> tr.shift) & tr.mask));
+    at[j] = t | (16 * (u ^ ((t >> tr.shift) & tr.mask)) << 4);
   }
   // K row (in rows of the pool; the V row is block_size further) of token
   // ts + lane % 32, tokens past the partition's last taking that one.
@@ -176,11 +173,12 @@ __global__ __launch_bounds__(64 * kTileWaves) void gen_tile_kernel(GenArgs a, Ge
   auto load = [&](uint32_t row, uint32_t dst) {
     uint32_t r[Sh::NI];
 #pragma unroll
-    for (int j = 0; j < Sh::NI; j++) r[j] = (uint32_t)__shfl((int)row, tok[j]);
+    for (int j = 0; j < Sh::NI; j++) r[j] = (uint32_t)__shfl((int)row, at[j] & 31);
 #pragma unroll
     for (int j = 0; j < Sh::NI; j++)
       if (j < ni)
-        tile_load_to_lds(head + (uint64_t)r[j] * row_bytes + uoff[j], dst + 1024u * j);
+        tile_load_to_lds(head + (uint64_t)r[j] * row_bytes + ((uint32_t)at[j] >> 4 & ~15u),
+                         dst + 1024u * j);
   };
 
   const int ts0 = t0 + attn::kTile * wave;
@@ -229,19 +227,48 @@ __global__ __launch_bounds__(64 * kTileWaves) void gen_tile_kernel(GenArgs a, Ge
     asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
     const uint32_t row = row_n;  // of the next tile
     const bool more = ts + kStride < t1;
+    // Operand reads run a batch ahead of the products (the scheduling
+    // barriers): left alone, the compiler reads each operand right before its
+    // product and waits out the LDS latency every time.
     f4_t s[2] = {f4_t{0.f, 0.f, 0.f, 0.f}, f4_t{0.f, 0.f, 0.f, 0.f}};
+    {
+      struct Batch {
+        h8_t qh[2], ql[2];
+        uint4 k[2][2];
+      } cur, nxt;
+      auto read = [&](int k0, Batch& f) {
 #pragma unroll
-    for (int ks = 0; ks < Sh::KS; ks++) {
-      const h8_t qh = lds.qop[ks * 64 + lane];
-      const h8_t ql = lds.qop[(Sh::KS + ks) * 64 + lane];
+        for (int i = 0; i < 2; i++) {
+          const int ks = k0 + i;
+          if (ks >= Sh::KS) break;
+          f.qh[i] = lds.qop[ks * 64 + lane];
+          f.ql[i] = lds.qop[(Sh::KS + ks) * 64 + lane];
 #pragma unroll
-      for (int tb = 0; tb < 2; tb++) {
-        uint4 kx = *reinterpret_cast<const uint4*>(kst + tr.at(16 * tb + l16, 4 * ks + grp));
-        // (past the head size: another token's features, whatever they hold)
-        if (8 * (4 * ks + grp) >= dph) kx = make_uint4(0u, 0u, 0u, 0u);
-        const h8_t k8 = __builtin_bit_cast(h8_t, kx);
-        s[tb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(k8, qh, s[tb], 0, 0, 0);
-        s[tb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(k8, ql, s[tb], 0, 0, 0);
+          for (int tb = 0; tb < 2; tb++)
+            f.k[i][tb] = *reinterpret_cast<const uint4*>(kst + tr.at(16 * tb + l16, 4 * ks + grp));
+        }
+      };
+      read(0, cur);
+#pragma unroll
+      for (int k0 = 0; k0 < Sh::KS; k0 += 2) {
+        if (k0 + 2 < Sh::KS) read(k0 + 2, nxt);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+          const int ks = k0 + i;
+          if (ks >= Sh::KS) break;
+#pragma unroll
+          for (int tb = 0; tb < 2; tb++) {
+            // (past the head size: another token's features, whatever they hold)
+            uint4 kx = cur.k[i][tb];
+            if (32 * ks + 32 > Sh::kLeast && 8 * (4 * ks + grp) >= dph)
+              kx = make_uint4(0u, 0u, 0u, 0u);
+            const h8_t k8 = __builtin_bit_cast(h8_t, kx);
+            s[tb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(k8, cur.qh[i], s[tb], 0, 0, 0);
+            s[tb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(k8, cur.ql[i], s[tb], 0, 0, 0);
+          }
+        }
+        cur = nxt;
       }
     }
     // Every operand read has returned (the products took them): the K tile
@@ -255,7 +282,7 @@ __global__ __launch_bounds__(64 * kTileWaves) void gen_tile_kernel(GenArgs a, Ge
       uint32_t bad = 0;
 #pragma unroll
       for (int j = 0; j < Sh::NI; j++)
-        if (j < ni && ts + tok[j] > wmin) {
+        if (j < ni && ts + (at[j] & 31) > wmin) {
           const uint4 v = *reinterpret_cast<const uint4*>(vst + 1024 * j + 16 * lane);
           bad |= attn::nonfinite_h2(v.x) | attn::nonfinite_h2(v.y) | attn::nonfinite_h2(v.z) |
                  attn::nonfinite_h2(v.w);
@@ -285,23 +312,45 @@ __global__ __launch_bounds__(64 * kTileWaves) void gen_tile_kernel(GenArgs a, Ge
         ps += p[4 * tb + i];
       }
     l_run = l_run * al + ps;
+    if (__builtin_amdgcn_ballot_w64(al != 1.f) != 0) {  // (a new max in some row)
 #pragma unroll
-    for (int db = 0; db < Sh::DB; db++) o[db] *= al;
+      for (int db = 0; db < Sh::DB; db++) o[db] *= al;
+    }
     if (!exact) {
-      h8_t ph, pl;
-      attn::split_h8(p, ph, pl);
       const int vt = 4 * grp + (l16 >> 2);
       const int vu = (l16 & 3) >> 1, vsub = 8 * (l16 & 1);
+      constexpr int kBatch = 4;
+      struct Batch {
+        s4_t v[kBatch][2];
+      } cur, nxt;
+      auto read = [&](int d0, Batch& f) {
 #pragma unroll
-      for (int db = 0; db < Sh::DB; db++) {
-        const s4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-            (lds_s4_t*)(vst + tr.at(vt, 2 * db + vu) + vsub));
-        const s4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-            (lds_s4_t*)(vst + tr.at(vt + 16, 2 * db + vu) + vsub));
-        const s4_t both[2] = {lo, hi};
-        const h8_t v8 = __builtin_bit_cast(h8_t, both);
-        o[db] = __builtin_amdgcn_mfma_f32_16x16x32_f16(v8, ph, o[db], 0, 0, 0);
-        o[db] = __builtin_amdgcn_mfma_f32_16x16x32_f16(v8, pl, o[db], 0, 0, 0);
+        for (int i = 0; i < kBatch; i++)
+#pragma unroll
+          for (int g = 0; g < 2; g++)
+            if (d0 + i < Sh::DB)
+              f.v[i][g] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                  (lds_s4_t*)(vst + tr.at(vt + 16 * g, 2 * (d0 + i) + vu) + vsub));
+      };
+      read(0, cur);
+      __builtin_amdgcn_sched_barrier(0);
+      h8_t ph, pl;
+      attn::split_h8(p, ph, pl);
+#pragma unroll
+      for (int d0 = 0; d0 < Sh::DB; d0 += kBatch) {
+        if (d0 + kBatch < Sh::DB) read(d0 + kBatch, nxt);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < kBatch; i++)
+          if (d0 + i < Sh::DB)
+            o[d0 + i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+                __builtin_bit_cast(h8_t, cur.v[i]), ph, o[d0 + i], 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < kBatch; i++)
+          if (d0 + i < Sh::DB)
+            o[d0 + i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+                __builtin_bit_cast(h8_t, cur.v[i]), pl, o[d0 + i], 0, 0, 0);
+        cur = nxt;
       }
     } else {
       // over the tokens each row sees; the weights go over the K tile
@@ -374,103 +423,9 @@ __global__ __launch_bounds__(64 * kTileWaves) void gen_tile_kernel(GenArgs a, Ge
           make_float2(x0 * inv, x1 * inv);
     } else {
       const size_t pr = ((size_t)kvh * a.R + gr) * a.n_parts + part;
-      attn::store_dev2(a.partials + pr * dph + d, x0, x1);
-      if (d == 0) attn::store_dev2(a.partials + n_acc + pr * 2, mx, l);
+      *reinterpret_cast<float2*>(a.partials + pr * dph + d) = make_float2(x0, x1);
+      if (d == 0) *reinterpret_cast<float2*>(a.partials + n_acc + pr * 2) = make_float2(mx, l);
     }
-  }
-  if (a.n_parts == 1) return;
-
-  // ---- the last workgroup of the (KV head, row group) combines ----------
-  // (device-scope stores, waited for before the arrival: store_dev2)
-  __builtin_amdgcn_s_waitcnt(0);
-  __syncthreads();
-  if (tid == 0) {
-    uint32_t* ctr = counters + (size_t)kvh * gridDim.z + rg;
-    const uint32_t prev =
-        __hip_atomic_fetch_add(ctr, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    lds.last = prev == (uint32_t)(a.n_parts - 1);
-    if (lds.last) __hip_atomic_store(ctr, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  }
-  __syncthreads();
-  if (!lds.last) return;
-  const int P = a.n_parts;
-  const uint32_t acc_bytes = (uint32_t)(n_acc * 4);
-  const uint32_t all_bytes = (uint32_t)((n_acc + (size_t)a.nkv * a.R * P * 2) * 4);
-  // a wave per row: lane p holds partition p's (max, sum)
-  for (int r = wave; r < nr; r += kTileWaves) {
-    const size_t row = (size_t)kvh * a.R + r0 + r;
-    const float2 ml = attn::load_dev8(
-        a.partials, all_bytes,
-        lane < P ? (uint32_t)((n_acc + (row * P + lane) * 2) * 4) : attn::kOutOfRange);
-    const float mx = attn::wave_max(lane < P ? ml.x : kNegInf);
-    const float w = lane < P ? part_weight(ml, mx) : 0.f;
-    const float l = attn::wave_sum(lane < P ? ml.y * w : 0.f);
-    if (lane < P) lds.wgt[r][lane] = w;
-    if (lane == 0) lds.wgt[r][attn::kStreamMaxParts] = 1.f / l;
-  }
-  __syncthreads();
-  // Thread -> (row, 4 features, slice of the partitions): few rows leave
-  // threads free, so up to 8 of them share a column's partitions (p = slice,
-  // slice + n_slices, ...) and meet in LDS, in slice order.
-  const int cols = dph / 4, items = nr * cols;
-  int n_slices = 1;
-  while (n_slices < 8 && 2 * n_slices * items <= 64 * kTileWaves && 2 * n_slices <= P) n_slices *= 2;
-  float4* meet = reinterpret_cast<float4*>(lds.st);
-  for (int i = tid; i < items * n_slices; i += 64 * kTileWaves) {
-    const int sl = i / items, it = i - sl * items;
-    const int r = it / cols, c = it - r * cols;
-    const size_t row = (size_t)kvh * a.R + r0 + r;
-    float4 sum = make_float4(0.f, 0.f, 0.f, 0.f);
-    for (int p0 = sl; p0 < P; p0 += 8 * n_slices) {
-      float4 v[8];
-#pragma unroll
-      for (int k = 0; k < 8; k++) {
-        const int p = p0 + k * n_slices;
-        v[k] = attn::load_dev16(a.partials, acc_bytes,
-                                p < P ? (uint32_t)(((row * P + p) * dph + 4 * c) * 4)
-                                      : attn::kOutOfRange);
-      }
-#pragma unroll
-      for (int k = 0; k < 8; k++) {
-        const int p = p0 + k * n_slices;
-        const float w = p < P ? lds.wgt[r][p] : 0.f;
-        sum.x += w * v[k].x;
-        sum.y += w * v[k].y;
-        sum.z += w * v[k].z;
-        sum.w += w * v[k].w;
-      }
-    }
-    if (n_slices > 1) {
-      meet[i] = sum;
-    } else {
-      const int gr = r0 + r;
-      const int m = gr / a.G, h = kvh * a.G + (gr - m * a.G);
-      const float inv = lds.wgt[r][attn::kStreamMaxParts];
-      float2* dst = reinterpret_cast<float2*>(a.out + (size_t)m * a.nh * dph + (size_t)h * dph +
-                                              4 * c);
-      dst[0] = make_float2(sum.x * inv, sum.y * inv);
-      dst[1] = make_float2(sum.z * inv, sum.w * inv);
-    }
-  }
-  if (n_slices == 1) return;
-  __syncthreads();
-  if (tid < items) {
-    const int r = tid / cols, c = tid - r * cols;
-    float4 sum = meet[tid];
-    for (int sl = 1; sl < n_slices; sl++) {
-      const float4 y = meet[sl * items + tid];
-      sum.x += y.x;
-      sum.y += y.y;
-      sum.z += y.z;
-      sum.w += y.w;
-    }
-    const int gr = r0 + r;
-    const int m = gr / a.G, h = kvh * a.G + (gr - m * a.G);
-    const float inv = lds.wgt[r][attn::kStreamMaxParts];
-    float2* dst =
-        reinterpret_cast<float2*>(a.out + (size_t)m * a.nh * dph + (size_t)h * dph + 4 * c);
-    dst[0] = make_float2(sum.x * inv, sum.y * inv);
-    dst[1] = make_float2(sum.z * inv, sum.w * inv);
   }
 }
 
@@ -478,6 +433,75 @@ template <bool ROPE>
 __global__ __launch_bounds__(kThreads) void gen_attn_kernel(GenArgs a, GenRope rp) {
   __shared__ GenLds lds;
   gen_unit<ROPE, kThreads>(a, &rp, blockIdx.x, blockIdx.y, blockIdx.z, lds);
+}
+
+// Log-sum-exp merge of the matrix-core form's partitions: four adjacent lanes
+// per (KV head, row, 4 features), lane s taking partitions s, s + 4, ...,
+// eight of them in flight; the lanes meet in a fixed order.  A kernel of its
+// own on all CUs: run by the last workgroup of a (KV head, row group), which
+// one CU's ~35 GB/s of partials bounds, calls measured slower from a few KB
+// on (5 queries of 16/8 heads of 256 over 3000 keys 24.8 us against 19.2;
+// one query of 32 heads of 96, the least partials, 16.9 against 17.3).
+__global__ __launch_bounds__(kThreads) void gen_tile_combine_kernel(GenArgs a) {
+  const int sub = threadIdx.x & 3;
+  const int cols = a.dph / 4;
+  const int64_t n = (int64_t)a.nkv * a.R * cols;
+  const int64_t item = ((int64_t)blockIdx.x * kThreads + threadIdx.x) >> 2;
+  const int64_t it = item < n ? item : n - 1;  // (whole waves for the exchanges)
+  const int64_t row = it / cols;               // kvh * R + rho
+  const int c = (int)(it - row * cols);
+  const int P = a.n_parts;
+  const float* acc = a.partials + row * P * a.dph + 4 * c;
+  const float2* mls =
+      reinterpret_cast<const float2*>(a.partials + (int64_t)a.nkv * a.R * P * a.dph) + row * P;
+  float mx = -__builtin_inff(), l = 0.f;
+  float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
+  for (int p0 = sub; p0 < P; p0 += 32) {
+    float2 ml[8];
+    float4 x[8];
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+      const int p = min(p0 + 4 * k, P - 1);  // (past the last: weight 0)
+      ml[k] = mls[p];
+      x[k] = *reinterpret_cast<const float4*>(acc + (int64_t)p * a.dph);
+    }
+    float top = mx;
+#pragma unroll
+    for (int k = 0; k < 8; k++) top = fmaxf(top, ml[k].x);
+    const float old = part_weight(make_float2(mx, l), top);
+    mx = top;
+    l *= old;
+    o.x *= old;
+    o.y *= old;
+    o.z *= old;
+    o.w *= old;
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+      const float w = p0 + 4 * k < P ? part_weight(ml[k], mx) : 0.f;
+      l += ml[k].y * w;
+      o.x += x[k].x * w;
+      o.y += x[k].y * w;
+      o.z += x[k].z * w;
+      o.w += x[k].w * w;
+    }
+  }
+  float top = fmaxf(mx, __shfl_xor(mx, 1));
+  top = fmaxf(top, __shfl_xor(top, 2));
+  const float w = part_weight(make_float2(mx, l), top);
+  float v[5] = {l * w, o.x * w, o.y * w, o.z * w, o.w * w};
+#pragma unroll
+  for (int i = 0; i < 5; i++) {
+    v[i] += __shfl_xor(v[i], 1);
+    v[i] += __shfl_xor(v[i], 2);
+  }
+  if (sub != 0 || item >= n) return;
+  const int h = (int)(row / a.R), rho = (int)(row - (int64_t)h * a.R);
+  const int m = rho / a.G, head = h * a.G + (rho - m * a.G);
+  const float inv = 1.f / v[0];
+  float2* d =
+      reinterpret_cast<float2*>(a.out + (size_t)m * a.nh * a.dph + (size_t)head * a.dph + 4 * c);
+  d[0] = make_float2(v[1] * inv, v[2] * inv);
+  d[1] = make_float2(v[3] * inv, v[4] * inv);
 }
 
 // Log-sum-exp merge of a row's partitions: workgroup (row rho, KV head).
@@ -538,7 +562,7 @@ size_t generic_partial_bytes(const GenPlan& p, int nkv, int R, int dph) {
 int generic_attention(uint16_t* pool, const int32_t* table, int kv_dim, int block_size,
                       const float* q, float* out, float* partials, int nh, int nkv, int dph,
                       int pos_base, int n_queries, const GenPlan& plan, const GenRope* rope,
-                      uint32_t* counters, hipStream_t stream) {
+                      bool tiles, hipStream_t stream) {
   if (dph > kMaxDph) return SDE_ERR_UNSUPPORTED;
   GenArgs a;
   a.pool = pool;
@@ -568,23 +592,28 @@ int generic_attention(uint16_t* pool, const int32_t* table, int kv_dim, int bloc
     if (st != SDE_OK) return st;
   }
   const dim3 grid(plan.n_parts, nkv, plan.row_groups);
-  if (counters) {
+  if (tiles) {
     const dim3 block(64 * kTileWaves);
     const int r = rope ? 1 : 0;
     if (dph <= 32)
-      gen_tile_kernel<32><<<grid, block, 0, stream>>>(a, rp, r, counters);
+      gen_tile_kernel<32><<<grid, block, 0, stream>>>(a, rp, r);
     else if (dph <= 64)
-      gen_tile_kernel<64><<<grid, block, 0, stream>>>(a, rp, r, counters);
+      gen_tile_kernel<64><<<grid, block, 0, stream>>>(a, rp, r);
     else if (dph <= 96)
-      gen_tile_kernel<96><<<grid, block, 0, stream>>>(a, rp, r, counters);
+      gen_tile_kernel<96><<<grid, block, 0, stream>>>(a, rp, r);
     else if (dph <= 128)
-      gen_tile_kernel<128><<<grid, block, 0, stream>>>(a, rp, r, counters);
+      gen_tile_kernel<128><<<grid, block, 0, stream>>>(a, rp, r);
     else if (dph <= 160)
-      gen_tile_kernel<160><<<grid, block, 0, stream>>>(a, rp, r, counters);
+      gen_tile_kernel<160><<<grid, block, 0, stream>>>(a, rp, r);
     else if (dph <= 192)
-      gen_tile_kernel<192><<<grid, block, 0, stream>>>(a, rp, r, counters);
+      gen_tile_kernel<192><<<grid, block, 0, stream>>>(a, rp, r);
     else
-      gen_tile_kernel<256><<<grid, block, 0, stream>>>(a, rp, r, counters);
+      gen_tile_kernel<256><<<grid, block, 0, stream>>>(a, rp, r);
+    const int st = launch_status();
+    if (st != SDE_OK || plan.n_parts == 1) return st;
+    const int64_t threads = (int64_t)nkv * a.R * dph;  // four per 4 features
+    gen_tile_combine_kernel<<<(unsigned)((threads + kThreads - 1) / kThreads), kThreads, 0,
+                              stream>>>(a);
     return launch_status();
   }
   if (rope)

@@ -43,7 +43,7 @@ size_t generic_partial_bytes(const GenPlan& p, int nkv, int R, int dph);
 int generic_attention(uint16_t* pool, const int32_t* table, int kv_dim, int block_size,
                       const float* q, float* out, float* partials, int nh, int nkv, int dph,
                       int pos_base, int n_queries, const GenPlan& plan,
-                      const GenRope* rope, uint32_t* counters, hipStream_t stream);
+                      const GenRope* rope, bool tiles, hipStream_t stream);
 
 }  // namespace gen
 }  // namespace sde

@@ -77,6 +77,13 @@ int parts_bound(int max_total_len) {
   return by_len < kStreamMaxParts ? by_len : kStreamMaxParts;
 }
 
+// The same for the generic path's matrix-core form, whose four waves take a
+// tile each: a partition holds at least 128 tokens.
+int tile_parts_bound(int max_total_len) {
+  const int by_len = (max_total_len + 127) / 128;
+  return by_len < kStreamMaxParts ? by_len : kStreamMaxParts;
+}
+
 // The plan of a call: 8-wave workgroups, one per CU.
 StreamPlan plan_for(int L_max, int nkv, int R, int n_cus) {
   return stream_plan8_spread(L_max, nkv, R, n_cus);
@@ -166,7 +173,10 @@ size_t sde_paged_attention_workspace_size(const sde_kv_cache* cache, int nh,
   if (!cache || nh < 1 || nkv < 1 || nh % nkv != 0 || n_queries < 1 || max_total_len < 1)
     return 0;
   const int R = n_queries * (nh / nkv);
-  return partial_bytes(nkv, R, parts_bound(max_total_len), dph);
+  const bool tiles = sde::gen::needs_generic(dph, cache->cfg.block_size) &&
+                     sde::gen::tile_serves(dph, cache->cfg.block_size, cache->cfg.pool_blocks);
+  return partial_bytes(nkv, R, tiles ? tile_parts_bound(max_total_len) : parts_bound(max_total_len),
+                       dph);
 }
 
 size_t sde_grid_attention_workspace_size(int nh, int nkv, int dph, int n_queries,
@@ -231,7 +241,7 @@ int run_attention(sde_kv_cache* cache, int layer, const float* d_q, float* d_out
       size_t most = SDE_NOALLOC_SCRATCH_BYTES;
       const int st = workspace_limit(cache, need, d_workspace, workspace_bytes, stream, &most);
       if (st != SDE_OK) return st;
-      gplan = sde::gen::tile_plan(L_max, nkv, R, dph, cache->n_cus, parts_bound(L_max), most);
+      gplan = sde::gen::tile_plan(L_max, nkv, R, dph, cache->n_cus, tile_parts_bound(L_max), most);
       need = sde::gen::generic_partial_bytes(gplan, nkv, R, dph);
     }
   } else {
@@ -286,8 +296,7 @@ int run_attention(sde_kv_cache* cache, int layer, const float* d_q, float* d_out
     return sde::gen::generic_attention(cache->pool, sde::layer_table(cache, layer),
                                        cache->cfg.kv_dim, cache->cfg.block_size, d_q, d_out,
                                        partials, nh, nkv, dph, pos_base, n_queries, gplan, grope,
-                                       tiles ? cache->d_counters : nullptr,
-                                       (hipStream_t)stream);
+                                       tiles, (hipStream_t)stream);
 
   AttnArgs a;
   a.src.pool = cache->pool;

@@ -70,7 +70,7 @@ def test_tile_form_matches_float64(gpu, oracle, nh, nkv, dph, bs, ctx, M):
     cache.free()
 
 
-@pytest.mark.parametrize("dph,bs", [(24, 16), (96, 16), (256, 7)])
+@pytest.mark.parametrize("dph,bs", [(24, 16), (80, 16), (96, 16), (200, 16), (256, 7)])
 def test_tile_form_hidden_nonfinite_rows(gpu, oracle, dph, bs):
     """Inf / NaN in V and NaN in K at a window position, and stale NaN past
     the window, reach only the queries that see them; fp16 padding features
