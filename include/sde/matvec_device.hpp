@@ -332,18 +332,27 @@ struct MvMfmaLds {
 // the item.  Scaling by a power of two commutes with every fp16 and fp32
 // rounding here, so the result equals the unscaled computation's wherever
 // that one is finite.  Every thread calls it; ends with a barrier.
-template <int WAVES>
+template <int MB, int WAVES>
 __device__ __forceinline__ void mv_row_scales(const MvArgs& a, const float* xl, int xrows,
                                               int r0, int r1, MvMfmaLds<WAVES>& L) {
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int lane = threadIdx.x & 63;
-  for (int m = 0; m < a.M; m++) {
-    float mx = 0.f;
-    if (wave < WAVES)
-      for (int i = wave * 64 + lane; i < xrows; i += WAVES * 64)
-        mx = fmaxf(mx, fabsf(xl ? xl[m * xrows + i] : a.x[(size_t)m * a.d_in + r0 + i]));
-    for (int off = 32; off > 0; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off));
-    if (wave < WAVES && lane == 0) L.xmax[wave][m] = mx;
+  // (all rows of a column of x together: their loads are in flight at once)
+  float mx[MB];
+#pragma unroll
+  for (int m = 0; m < MB; m++) mx[m] = 0.f;
+  if (wave < WAVES)
+    for (int i = wave * 64 + lane; i < xrows; i += WAVES * 64)
+#pragma unroll
+      for (int m = 0; m < MB; m++) {
+        const int mm = m < a.M ? m : 0;
+        mx[m] = fmaxf(mx[m],
+                      fabsf(xl ? xl[mm * xrows + i] : a.x[(size_t)mm * a.d_in + r0 + i]));
+      }
+#pragma unroll
+  for (int m = 0; m < MB; m++) {
+    for (int off = 32; off > 0; off >>= 1) mx[m] = fmaxf(mx[m], __shfl_xor(mx[m], off));
+    if (wave < WAVES && lane == 0 && m < a.M) L.xmax[wave][m] = mx[m];
   }
   __syncthreads();
   if ((int)threadIdx.x < a.M) {
@@ -360,17 +369,20 @@ __device__ __forceinline__ void mv_row_scales(const MvArgs& a, const float* xl, 
   __syncthreads();
 }
 __device__ __forceinline__ int mv_staged(int r, int u) { return r * (kCols * 2) + 16 * (u ^ (r & 15)); }
+// Row of x and W of element q of the lane's x operand, in the batch at rbase.
 template <int WAVES>
-__device__ __forceinline__ void mv_x_operand(const MvArgs& a, const float* xl, int xrows, int r0,
-                                             int r1, int rbase, int lane, float sc, mv_h4& xh,
+__device__ __forceinline__ int mv_x_row(int rbase, int lane, int q) {
+  const int lr = 4 * (lane >> 4) + q;
+  return rbase + (lr >> 1) * WAVES * kRowPhases + (lr & 1);
+}
+template <int WAVES>
+__device__ __forceinline__ void mv_x_operand(const MvArgs& a, const float (&x)[4], int r1,
+                                             int rbase, int lane, float sc, mv_h4& xh,
                                              mv_h4& xo) {
-  const int m = lane & 15, g = lane >> 4;
 #pragma unroll
   for (int q = 0; q < 4; q++) {
-    const int lr = 4 * g + q;
-    const int row = rbase + (lr >> 1) * WAVES * kRowPhases + (lr & 1);
-    float v = 0.f;
-    if (m < a.M && row < r1) v = (xl ? xl[m * xrows + row - r0] : a.x[(size_t)m * a.d_in + row]) * sc;
+    const bool live = (lane & 15) < a.M && mv_x_row<WAVES>(rbase, lane, q) < r1;
+    float v = live ? x[q] * sc : 0.f;
     asm("" : "+v"(v));  // rounded once: hi = fp16(v), lo = fp16(v - hi)
     const _Float16 h = (_Float16)v;
     xh[q] = h;
@@ -394,6 +406,59 @@ __device__ __forceinline__ void mv_mfma_batch(const char* st, int lane, mv_h4 xh
     const mv_h4 w = __builtin_bit_cast(mv_h4, s);
     c[cb] = __builtin_amdgcn_mfma_f32_16x16x16f16(w, xh, c[cb], 0, 0, 0);
     c[cb] = __builtin_amdgcn_mfma_f32_16x16x16f16(w, xo, c[cb], 0, 0, 0);
+  }
+}
+
+// A wave's rows of a range, on the matrix cores.  Each batch's loads of W,
+// and of x where the range's x is not staged in LDS (XL), are issued before
+// the multiplication of the batch before it, x's first: loaded where they
+// are used, x's values (a wide head has one range, whose x outgrows the
+// staging area) came back behind the next batch of W, and every wave drained
+// its loads twice per two batches (5 rows of a 4096 x 128256 head and the
+// sampling behind it: 262 -> 213 us, of which the weights take 180 at the
+// rate of a streaming read).
+template <int WAVES, bool XL>
+__device__ __forceinline__ void mv_mfma_stream(const MvArgs& a, const MvRows& rows,
+                                               const float* xl, int xrows, int first, int lane,
+                                               int rp, int lc, float sc, char* st,
+                                               mv_f4 (&c)[kColBlocks]) {
+  constexpr int U = kUnroll;
+  constexpr int step = WAVES * U * kRowPhases;  // rows per batch of the workgroup
+  const int r0 = rows.r0, r1 = rows.r1;
+  const size_t xm = (size_t)min(lane & 15, a.M - 1);
+  struct Batch {
+    float x[4];
+    uint4 w[U];
+  } ba, bb;
+  // (past the range: x's last row, and zeros for W without a memory access)
+  auto load = [&](int r, Batch& b) {
+    const int rc = min(r, r1);
+    if constexpr (!XL) {
+#pragma unroll
+      for (int q = 0; q < 4; q++)
+        b.x[q] = a.x[xm * a.d_in + min(mv_x_row<WAVES>(rc, lane, q), r1 - 1)];
+    }
+    mv_load_batch<WAVES, U>(rows, rc, b.w);
+  };
+  auto multiply = [&](int r, Batch& b) {
+    if constexpr (XL) {
+#pragma unroll
+      for (int q = 0; q < 4; q++)
+        b.x[q] = xl[xm * xrows + min(mv_x_row<WAVES>(r, lane, q), r1 - 1) - r0];
+    }
+    mv_h4 xh, xo;
+    mv_x_operand<WAVES>(a, b.x, r1, r, lane, sc, xh, xo);
+    mv_stage<U>(st, rp, lc, b.w);  // (a wave's LDS operations complete in order)
+    mv_mfma_batch(st, lane, xh, xo, c);
+  };
+  load(first, ba);
+  for (int r = first; r < r1; r += 2 * step) {
+    load(r + step, bb);
+    __builtin_amdgcn_sched_barrier(0);
+    multiply(r, ba);
+    load(r + 2 * step, ba);
+    __builtin_amdgcn_sched_barrier(0);
+    if (r + step < r1) multiply(r + step, bb);
   }
 }
 
@@ -439,7 +504,7 @@ __device__ __forceinline__ void mv_item(const MvArgs& a, int ct, int ks, Lds& L)
     __syncthreads();
     xl = lds.xs;
   }
-  if constexpr (MFMA) mv_row_scales<WAVES>(a, xl, xrows, r0, r1, L);
+  if constexpr (MFMA) mv_row_scales<MB, WAVES>(a, xl, xrows, r0, r1, L);
 
   if (wave < WAVES) {
     // Row blocks of kRowPhases rows: the wave takes blocks wave, wave +
@@ -453,20 +518,10 @@ __device__ __forceinline__ void mv_item(const MvArgs& a, int ct, int ks, Lds& L)
     if constexpr (MFMA) {
       char* st = reinterpret_cast<char*>(L.wst[wave]);
       const float sc = L.xscale[min(lane & 15, a.M - 1)];  // this lane's row of x
-      for (int r = first; r < r1; r += 2 * step) {
-        uint4 wa[U], wb[U];
-        mv_load_batch<WAVES, U>(rows, r, wa);
-        mv_load_batch<WAVES, U>(rows, r + step, wb);
-        mv_h4 xh, xo;
-        mv_x_operand<WAVES>(a, xl, xrows, r0, r1, r, lane, sc, xh, xo);
-        mv_stage<U>(st, rp, lc, wa);
-        mv_mfma_batch(st, lane, xh, xo, cm);
-        if (r + step < r1) {
-          mv_x_operand<WAVES>(a, xl, xrows, r0, r1, r + step, lane, sc, xh, xo);
-          mv_stage<U>(st, rp, lc, wb);  // (a wave's LDS operations complete in order)
-          mv_mfma_batch(st, lane, xh, xo, cm);
-        }
-      }
+      if (xl)
+        mv_mfma_stream<WAVES, true>(a, rows, xl, xrows, first, lane, rp, lc, sc, st, cm);
+      else
+        mv_mfma_stream<WAVES, false>(a, rows, nullptr, xrows, first, lane, rp, lc, sc, st, cm);
     } else {
     for (int r = first; r < r1; r += 2 * step) {
       uint4 wa[U], wb[U];

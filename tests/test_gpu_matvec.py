@@ -311,3 +311,27 @@ def test_grid_matvec_errors_write_nothing(gpu, mvdev):
     assert (st == N.SDE_ERR_UNSUPPORTED).all() and torch.isnan(ot).all()
     st = _grid_mv(mvdev, gpu, xt, Wt, ot, 17, 4096, 4096, 0, 8, 512, ws)
     assert (st == N.SDE_ERR_INVALID_ARGUMENT).all() and torch.isnan(ot).all()
+
+
+@pytest.mark.parametrize("M,d_in,d_out", [
+    (3, 1543, 33032),   # one odd row range per tile, a partial last tile and batch
+    (5, 1024, 40960),   # whole batches only
+    (8, 4099, 33288),   # an odd number of batch pairs
+    (11, 600, 65544),   # two passes of unequal rows; the second's x is staged
+    (4, 1030, 33032),   # range just past the staging area
+])
+def test_matvec_wide_heads_read_x_from_memory(gpu, M, d_in, d_out):
+    """Matrices wide enough for one row range per column tile, whose x does
+    not fit the staging area: x comes from memory, a batch ahead."""
+    case_banner("matvec wide head", M, d_in, d_out)
+    g = torch.Generator(device=gpu).manual_seed(d_in + M)
+    x = torch.randn(M, d_in, generator=g, device=gpu)
+    x[-1, -1] = 3e5  # past the fp16 range, in the last row of the last batch
+    W = (0.05 * torch.randn(d_in, d_out, generator=g, device=gpu)).half()
+    got = matvec(x, W)
+    x64 = x.double()
+    for c in range(0, d_out, 8192):
+        w = W[:, c:c + 8192].double()
+        err = (got[:, c:c + 8192].double() - x64 @ w).abs()
+        assert bool((err <= MV_TOL * (x64.abs() @ w.abs())).all())
+    assert torch.equal(matvec(x, W), got)
