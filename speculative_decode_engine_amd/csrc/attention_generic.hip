@@ -56,7 +56,7 @@ __global__ __launch_bounds__(kThreads) void gen_rope_append_kernel(GenArgs a, Ge
 // Bound by the latency of a few tiles in turn and, as they grow, by memory.
 // Measured on MI355X, us per layer, fp32 form / this: decode over 3000 keys,
 // 32 KV heads of 96, 188 + 13 (combine) / 17.3 in all; a 5-query window over
-// 4000 keys, 16/8 heads of 256, RoPE of q included, 193 + 15 / 28.  Errors
+// 4000 keys, 16/8 heads of 256, RoPE and the append included, 212 / 26.  Errors
 // against float64 fell too (4.7e-7 -> 3.0e-7, 6.5e-7 -> 4.2e-7 of the
 // output's norm): shorter sums.
 // DPHP: the head size rounded up to a multiple of 32.
@@ -181,6 +181,25 @@ __global__ __launch_bounds__(64 * kTileWaves) void gen_tile_kernel(GenArgs a, Ge
                          dst + 1024u * j);
   };
 
+  // ---- RoPE's operands: thread -> pairs (row, j) of q, features j and j +
+  // dph / 2.  Their loads go out before the block table's, whose wait covers
+  // them; behind the tile loads they would come back after the tiles.
+  constexpr int kPairs = kTileRows * (DPHP / 2) / (64 * kTileWaves);
+  const int half = dph / 2, n_pairs = nr * half;
+  float qa[kPairs], qb[kPairs], qf[kPairs];
+  if (use_rope) {
+#pragma unroll
+    for (int k = 0; k < kPairs; k++) {
+      const int i = min(tid + 64 * kTileWaves * k, n_pairs - 1);
+      const int r = i / half, j = i - r * half;
+      const int m = (r0 + r) / a.G, h = kvh * a.G + (r0 + r - m * a.G);
+      const float* qrow = a.q + (size_t)m * a.nh * dph + (size_t)h * dph;
+      qa[k] = qrow[j];
+      qb[k] = qrow[j + half];
+      qf[k] = rp.inv_freq[j];
+    }
+  }
+
   const int ts0 = t0 + attn::kTile * wave;
   constexpr int kStride = attn::kTile * kTileWaves;
   uint32_t row_n = 0;  // the rows of the next tile to load
@@ -191,29 +210,50 @@ __global__ __launch_bounds__(64 * kTileWaves) void gen_tile_kernel(GenArgs a, Ge
     load(row + (uint32_t)a.bs, k_off + Sh::TILEB);
   }
 
-  // ---- q operand: thread -> units of 8 features of a row ----------------
+  // ---- q operand, while the tiles are on their way ----------------------
   // (hi part of k-step ks at qop[64 ks + lane], lo behind all of them; lane =
-  // row + 16 (unit % 4))
+  // row + 16 (unit % 4)): units of 8 features, with RoPE the padding alone --
+  // one angle per pair and thread (a unit per thread formed both of a pair's
+  // elements' angles, 16 in turn at head size 256: 5-query window over 4000
+  // keys, 16/8 heads, the whole layer 29.8 -> 26.1 us)
   for (int i = tid; i < kTileRows * (DPHP / 8); i += 64 * kTileWaves) {
     const int r = i / (DPHP / 8), u = i - r * (DPHP / 8);
+    const bool some = r < nr && u < U;
+    if (some && use_rope) continue;
     float x[8];
 #pragma unroll
     for (int e = 0; e < 8; e++) x[e] = 0.f;
-    if (r < nr && u < U) {
+    if (some) {
       const int gr = r0 + r;
       const int m = gr / a.G, h = kvh * a.G + (gr - m * a.G);
       const float* qrow = a.q + (size_t)m * a.nh * dph + (size_t)h * dph;
 #pragma unroll
-      for (int e = 0; e < 8; e++) {
-        const int d = 8 * u + e;
-        x[e] = (use_rope ? rope_elem(qrow, d, dph, a.pos_base + m, rp) : qrow[d]) * a.qscale;
-      }
+      for (int e = 0; e < 8; e++) x[e] = qrow[8 * u + e] * a.qscale;
     }
     h8_t hi, lo;
     attn::split_h8(x, hi, lo);
     const int at = (u >> 2) * 64 + (u & 3) * 16 + r;
     lds.qop[at] = hi;
     lds.qop[Sh::KS * 64 + at] = lo;
+  }
+  if (use_rope) {
+    auto put = [&](int r, int d, float v) {
+      const int u = d >> 3, at = (u >> 2) * 64 + (u & 3) * 16 + r;
+      asm("" : "+v"(v));  // (rounded once, as in split_h8)
+      const _Float16 h = (_Float16)v;
+      reinterpret_cast<_Float16*>(&lds.qop[at])[d & 7] = h;
+      reinterpret_cast<_Float16*>(&lds.qop[Sh::KS * 64 + at])[d & 7] = (_Float16)(v - (float)h);
+    };
+#pragma unroll
+    for (int k = 0; k < kPairs; k++) {
+      const int i = tid + 64 * kTileWaves * k;
+      if (i >= n_pairs) break;
+      const int r = i / half, j = i - r * half;
+      float sn, cs;
+      sincosf(((float)(a.pos_base + (r0 + r) / a.G) / rp.pos_div) * qf[k], &sn, &cs);
+      put(r, j, (qa[k] * cs - qb[k] * sn) * a.qscale);
+      put(r, j + half, (qa[k] * sn + qb[k] * cs) * a.qscale);
+    }
   }
   __syncthreads();
 

@@ -93,3 +93,52 @@ def test_tile_form_hidden_nonfinite_rows(gpu, oracle, dph, bs):
     # (KV head 0's rows hold the NaN key: not finite from query 4 on)
     assert not np.isfinite(out[4:, :dph]).any()
     cache.free()
+
+
+def _rotated(q, heads, dph, ctx, theta):
+    """Rotate-half RoPE in 64 bits at the path's own fp32 angles."""
+    half = dph // 2
+    inv = np.exp(-np.log(theta) * 2.0 * np.arange(half) / dph).astype(np.float32)
+    pos = np.arange(ctx, ctx + q.shape[0], dtype=np.float32)
+    ang = (pos[:, None] * inv[None, :]).astype(np.float64)[:, None, :]
+    x = q.astype(np.float64).reshape(q.shape[0], heads, dph)
+    a, b = x[..., :half], x[..., half:]
+    y = np.concatenate([a * np.cos(ang) - b * np.sin(ang), a * np.sin(ang) + b * np.cos(ang)], -1)
+    return y.reshape(q.shape).astype(np.float32)
+
+
+@pytest.mark.parametrize("nh,nkv,dph,bs,ctx,M", [
+    (1, 1, 8, 16, 0, 1),       # four pairs in all
+    (3, 1, 24, 16, 130, 1),    # halves that are no multiple of 8
+    (16, 1, 32, 16, 500, 1),   # a full group of 16 rows
+    (17, 1, 40, 16, 500, 1),   # one row past it
+    (7, 1, 96, 16, 300, 5),    # groups that begin inside a query's heads
+    (4, 4, 120, 12, 700, 9),
+    (12, 4, 64, 12, 700, 3),   # head size 64 with a block size of this form
+    (16, 8, 256, 16, 3000, 5),
+    (32, 2, 256, 16, 257, 2),  # 32 rows, all pairs of a thread in use
+    (24, 2, 200, 16, 900, 9),  # 108 rows, the last group not full
+])
+def test_tile_form_rope_equals_rotated_queries(gpu, nh, nkv, dph, bs, ctx, M):
+    """The call with RoPE against the same call on queries rotated beforehand."""
+    case_banner("tile form, rope", nh, nkv, dph, bs, ctx, M)
+    cache, K, V, rng = build_layer(nh, nkv, dph, bs, ctx, M, -(-(ctx + M) // bs) + 9, dph + ctx)
+    q = W.queries(rng, M, nh, dph)
+    k = rng.standard_normal((M, nkv * dph)).astype(np.float32)
+    v = rng.standard_normal((M, nkv * dph)).astype(np.float32)
+    got = cache.rope_append_attention(0, *(torch.from_numpy(t).cuda() for t in (q, k, v)), nh,
+                                      nkv, dph, ctx, theta=10000.0)
+    # (the window's keys are in the cache now, rotated)
+    want = cache.attention(0, torch.from_numpy(_rotated(q, nh, dph, ctx, 10000.0)).cuda(), nh,
+                           nkv, dph, ctx)
+    keys, _ = cache.read(0, 0, ctx + M)
+    # An element's rotation is within 2^-21 of its pair's norm (sine, cosine,
+    # two products and a sum in fp32), so a logit within 2^-21 |q| |k| /
+    # sqrt(dph) and a softmax mean within twice that of the largest |v|; both
+    # calls' own sums add 2^-19.
+    qn = float(np.linalg.norm(q.reshape(-1, dph), axis=1).max())
+    kn = float(keys.reshape(-1, dph).norm(dim=1).max())
+    vmax = max(float(np.abs(V).max()) if ctx else 0.0, float(np.abs(v).max()))
+    bound = (2.0 ** -20 * qn * kn / np.sqrt(dph) + 2.0 ** -19) * vmax
+    assert float((got - want).abs().max()) <= bound
+    cache.free()
