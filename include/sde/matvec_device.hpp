@@ -414,9 +414,10 @@ __device__ __forceinline__ void mv_mfma_batch(const char* st, int lane, mv_h4 xh
 // the multiplication of the batch before it, x's first: loaded where they
 // are used, x's values (a wide head has one range, whose x outgrows the
 // staging area) came back behind the next batch of W, and every wave drained
-// its loads twice per two batches (5 rows of a 4096 x 128256 head and the
-// sampling behind it: 262 -> 213 us, of which the weights take 180 at the
-// rate of a streaming read).
+// its loads twice per two batches (measured on MI355X, us, without / with:
+// 5 rows of a 4096 x 128256 head 227 / 181, of which the weights take 180 at
+// the rate of a streaming read, of 2048 x 32000 39.1 / 30.1; staged x, 5 rows
+// of 14336 x 4096 44.9 / 34.4, of 4096 x 4096 23.8 / 21.6).
 template <int WAVES, bool XL>
 __device__ __forceinline__ void mv_mfma_stream(const MvArgs& a, const MvRows& rows,
                                                const float* xl, int xrows, int first, int lane,
