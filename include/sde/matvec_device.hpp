@@ -196,19 +196,24 @@ __device__ __forceinline__ void mv_load_batch(const MvRows& t, int r, uint4 (&w)
 // row blocks are wave-uniform) and picked per lane group.
 // x of the lane's row: from xl (the row range staged in LDS as
 // [m][row - r0], `rows` long) when given, else a scalar load per row phase
-// picked per lane group (a single row of x: the whole batch's scalars are
-// loaded ahead).
+// picked per lane group (one or two rows of x: the whole batch's scalars are
+// loaded ahead; two rows of a 4096 x 128256 head, us, without / with:
+// 314 / 174).
 template <int MB, int WAVES, int U, bool FULL>
 __device__ __forceinline__ void mv_fma_batch(const struct MvArgs& a, int r, int r0, int r1,
                                              int rp, const float* xl, int rows,
                                              const uint4 (&w)[U], float (&acc)[MB][8]) {
-  float xs[U][kRowPhases];
-  if (MB == 1 && !xl) {
+  constexpr bool kAhead = MB <= 2;
+  float xs[kAhead ? MB : 1][U][kRowPhases];
+  if (kAhead && !xl) {
 #pragma unroll
-    for (int u = 0; u < U; u++)
+    for (int m = 0; m < (kAhead ? MB : 1); m++)
 #pragma unroll
-      for (int p = 0; p < kRowPhases; p++)
-        xs[u][p] = a.x[min(r + u * WAVES * kRowPhases + p, a.d_in - 1)];
+      for (int u = 0; u < U; u++)
+#pragma unroll
+        for (int p = 0; p < kRowPhases; p++)
+          xs[m][u][p] = a.x[(size_t)min(m, a.M - 1) * a.d_in +
+                            min(r + u * WAVES * kRowPhases + p, a.d_in - 1)];
   }
   // LDS-staged x: the values of UP row blocks are read up front, so their
   // LDS round trips overlap instead of sitting in the multiply-add chain
@@ -233,10 +238,10 @@ __device__ __forceinline__ void mv_fma_batch(const struct MvArgs& a, int r, int 
         float xv;
         if (xl) {
           xv = xpre[u % UP][m];
-        } else if (MB == 1) {
-          xv = xs[u][0];
+        } else if (kAhead) {
+          xv = xs[kAhead ? m : 0][u][0];
 #pragma unroll
-          for (int p = 1; p < kRowPhases; p++) xv = rp == p ? xs[u][p] : xv;
+          for (int p = 1; p < kRowPhases; p++) xv = rp == p ? xs[kAhead ? m : 0][u][p] : xv;
         } else {
           xv = a.x[(size_t)m * a.d_in + min(rb + rp, r1 - 1)];
         }

@@ -319,6 +319,7 @@ def test_grid_matvec_errors_write_nothing(gpu, mvdev):
     (8, 4099, 33288),   # an odd number of batch pairs
     (11, 600, 65544),   # two passes of unequal rows; the second's x is staged
     (4, 1030, 33032),   # range just past the staging area
+    (2, 4099, 33032),   # two rows, on the VALU
 ])
 def test_matvec_wide_heads_read_x_from_memory(gpu, M, d_in, d_out):
     """Matrices wide enough for one row range per column tile, whose x does
