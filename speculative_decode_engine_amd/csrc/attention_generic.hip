@@ -51,7 +51,10 @@ __global__ __launch_bounds__(kThreads) void gen_rope_append_kernel(GenArgs a, Ge
 //    barrier;
 //  * logits K . Q^T and output V^T . P^T are 16x16x32 fp16 MFMA over the
 //    head size padded to 32, q and the weights as fp16 hi + lo pairs, sums
-//    in fp32 (the layouts of attention_device.hpp's tile path);
+//    in fp32 (the layouts of attention_device.hpp's tile path).  A row of q
+//    is scaled by a power of two into fp16's range first and its logits back
+//    (any finite q works, and a lo part never loses bits to fp16's least
+//    exponent);
 //  * the waves' sums meet in LDS, the partitions' in a combine kernel.
 // Bound by the latency of a few tiles in turn and, as they grow, by memory.
 // Measured on MI355X, us per layer, fp32 form / this: decode over 3000 keys,
@@ -77,6 +80,11 @@ struct TileShape {
   static constexpr int WAVEB = 2 * TILEB;                  // a wave's K and V tile
   // the next smaller form's head size: features below it always exist
   static constexpr int kLeast = DPHP == 256 ? 192 : DPHP - 32;
+  // fp16 parts of q: two carry 22-23 of its 24 bits, which is less than the
+  // rounding of a long sum of products and more than that of a short one
+  // (q x 16 at head size 32, largest error over the output's: fp32 form
+  // 1.7e-6, two parts 2.7e-6, three 0.8e-6; at 48 5.3e-6, 1.2e-6, 1.2e-6).
+  static constexpr int QP = DPHP <= 32 ? 3 : 2;
 };
 
 template <int DPHP>
@@ -85,7 +93,8 @@ struct TileLds {
   // (+ 1 KiB: a feature block past the head size is read, and dropped, from
   // behind the tile's last row)
   char st[kTileWaves * Sh::WAVEB + 1024] __attribute__((aligned(16)));
-  h8_t qop[2 * Sh::KS * 64];
+  h8_t qop[Sh::QP * Sh::KS * 64];
+  int qexp[kTileRows];  // rows of q: the exponent of the power of two on it
   float2 ml[kTileWaves][kTileRows];
   static_assert(kTileRows * DPHP * 4 <= Sh::WAVEB, "a wave's sums fit its tiles");
 };
@@ -118,6 +127,20 @@ struct TileRow {
 __device__ __forceinline__ float part_weight(float2 ml, float mx) {
   if (ml.x == -__builtin_inff()) return ml.y == 0.f ? 0.f : 1.f;
   return __builtin_amdgcn_exp2f(ml.x - mx);
+}
+
+// Max over the 16 lanes of a wave's row, returned to all of them.
+__device__ __forceinline__ float max16(float x) {
+#define SDE_ROR(n)                                                                          \
+  x = fmaxf(x, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(                       \
+                                             0, __builtin_bit_cast(int, x), 0x120 + n, 0xf, \
+                                             0xf, false)))
+  SDE_ROR(8);
+  SDE_ROR(4);
+  SDE_ROR(2);
+  SDE_ROR(1);
+#undef SDE_ROR
+  return x;
 }
 
 template <int DPHP>
@@ -181,23 +204,47 @@ __global__ __launch_bounds__(64 * kTileWaves) void gen_tile_kernel(GenArgs a, Ge
                          dst + 1024u * j);
   };
 
-  // ---- RoPE's operands: thread -> pairs (row, j) of q, features j and j +
-  // dph / 2.  Their loads go out before the block table's, whose wait covers
+  // ---- q: thread -> row tid / 16, units (tid % 16) + 16 n; with RoPE
+  // instead the wave -> a run of rows, the lane -> pairs, features j and j +
+  // dph / 2.  These loads go out before the block table's, whose wait covers
   // them; behind the tile loads they would come back after the tiles.
-  constexpr int kPairs = kTileRows * (DPHP / 2) / (64 * kTileWaves);
-  const int half = dph / 2, n_pairs = nr * half;
-  float qa[kPairs], qb[kPairs], qf[kPairs];
+  auto q_row = [&](int r) {
+    const int m = (r0 + r) / a.G, h = kvh * a.G + (r0 + r - m * a.G);
+    return a.q + (size_t)m * a.nh * dph + (size_t)h * dph;
+  };
+  constexpr int kUnits = (DPHP / 8 + 15) / 16;
+  const int qr = tid >> 4, qs = tid & 15;
+  float x[kUnits][8];
+#pragma unroll
+  for (int n = 0; n < kUnits; n++)
+#pragma unroll
+    for (int e = 0; e < 8; e++) x[n][e] = 0.f;
+  constexpr int kWaveRows = kTileRows / kTileWaves, kPairs = (DPHP / 2 + 63) / 64;
+  const int half = dph / 2;
+  const int wave_rows = (nr + kTileWaves - 1) / kTileWaves, wr0 = wave * wave_rows;
+  float qa[kWaveRows][kPairs], qb[kWaveRows][kPairs], qf[kPairs];
   if (use_rope) {
 #pragma unroll
-    for (int k = 0; k < kPairs; k++) {
-      const int i = min(tid + 64 * kTileWaves * k, n_pairs - 1);
-      const int r = i / half, j = i - r * half;
-      const int m = (r0 + r) / a.G, h = kvh * a.G + (r0 + r - m * a.G);
-      const float* qrow = a.q + (size_t)m * a.nh * dph + (size_t)h * dph;
-      qa[k] = qrow[j];
-      qb[k] = qrow[j + half];
-      qf[k] = rp.inv_freq[j];
+    for (int k = 0; k < kPairs; k++) qf[k] = rp.inv_freq[min(lane + 64 * k, half - 1)];
+#pragma unroll
+    for (int i = 0; i < kWaveRows; i++) {
+      if (i >= wave_rows || wr0 + i >= nr) break;
+      const float* qrow = wave_uniform(q_row(wr0 + i));
+#pragma unroll
+      for (int k = 0; k < kPairs; k++) {
+        const int j = min(lane + 64 * k, half - 1);
+        qa[i][k] = qrow[j];
+        qb[i][k] = qrow[j + half];
+      }
     }
+  } else if (qr < nr) {
+    const float* qrow = q_row(qr);
+#pragma unroll
+    for (int n = 0; n < kUnits; n++)
+      if (qs + 16 * n < U) {
+#pragma unroll
+        for (int e = 0; e < 8; e++) x[n][e] = qrow[8 * (qs + 16 * n) + e];
+      }
   }
 
   const int ts0 = t0 + attn::kTile * wave;
@@ -211,51 +258,91 @@ __global__ __launch_bounds__(64 * kTileWaves) void gen_tile_kernel(GenArgs a, Ge
   }
 
   // ---- q operand, while the tiles are on their way ----------------------
-  // (hi part of k-step ks at qop[64 ks + lane], lo behind all of them; lane =
-  // row + 16 (unit % 4)): units of 8 features, with RoPE the padding alone --
-  // one angle per pair and thread (a unit per thread formed both of a pair's
-  // elements' angles, 16 in turn at head size 256: 5-query window over 4000
-  // keys, 16/8 heads, the whole layer 29.8 -> 26.1 us)
-  for (int i = tid; i < kTileRows * (DPHP / 8); i += 64 * kTileWaves) {
-    const int r = i / (DPHP / 8), u = i - r * (DPHP / 8);
-    const bool some = r < nr && u < U;
-    if (some && use_rope) continue;
-    float x[8];
+  // (part p of k-step ks at qop[(p KS + ks) 64 + lane]; lane = row +
+  // 16 (unit % 4)).  A row's largest element is brought to [2^14, 2^15) by a
+  // power of two (2^exponent and its inverse are normal numbers; zero, Inf
+  // and NaN take 2^15), a rotated one thus below 2^15.5.
+  auto exponent = [](float mx) { return min(15 - __builtin_amdgcn_frexp_expf(mx), 126); };
+  {
+    float mx = 0.f;
 #pragma unroll
-    for (int e = 0; e < 8; e++) x[e] = 0.f;
-    if (some) {
-      const int gr = r0 + r;
-      const int m = gr / a.G, h = kvh * a.G + (gr - m * a.G);
-      const float* qrow = a.q + (size_t)m * a.nh * dph + (size_t)h * dph;
+    for (int n = 0; n < kUnits; n++)
 #pragma unroll
-      for (int e = 0; e < 8; e++) x[e] = qrow[8 * u + e] * a.qscale;
+      for (int e = 0; e < 8; e++) {
+        x[n][e] *= a.qscale;
+        mx = fmaxf(mx, fabsf(x[n][e]));
+      }
+    const int qe = exponent(max16(mx));
+    if (qs == 0 && !(use_rope && qr < nr)) lds.qexp[qr] = qe;
+#pragma unroll
+    for (int n = 0; n < kUnits; n++) {
+      const int u = qs + 16 * n;
+      if (u >= DPHP / 8 || (use_rope && qr < nr && u < U)) continue;
+      const int at = (u >> 2) * 64 + (u & 3) * 16 + qr;
+#pragma unroll
+      for (int e = 0; e < 8; e++) x[n][e] = ldexpf(x[n][e], qe);
+#pragma unroll
+      for (int p = 0; p < Sh::QP; p++) {
+        h8_t part;
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+          asm("" : "+v"(x[n][e]));  // (rounded once, as in split_h8)
+          part[e] = (_Float16)x[n][e];
+          x[n][e] -= (float)part[e];
+        }
+        lds.qop[p * Sh::KS * 64 + at] = part;
+      }
     }
-    h8_t hi, lo;
-    attn::split_h8(x, hi, lo);
-    const int at = (u >> 2) * 64 + (u & 3) * 16 + r;
-    lds.qop[at] = hi;
-    lds.qop[Sh::KS * 64 + at] = lo;
   }
+  // With RoPE one angle per pair and query: the rows of a query (its heads)
+  // follow each other in the wave's run (an angle per element: 5-query window
+  // over 4000 keys, 16/8 heads of 256, the whole layer 29.8 us; this 26.4).
   if (use_rope) {
-    auto put = [&](int r, int d, float v) {
-      const int u = d >> 3, at = (u >> 2) * 64 + (u & 3) * 16 + r;
-      asm("" : "+v"(v));  // (rounded once, as in split_h8)
-      const _Float16 h = (_Float16)v;
-      reinterpret_cast<_Float16*>(&lds.qop[at])[d & 7] = h;
-      reinterpret_cast<_Float16*>(&lds.qop[Sh::KS * 64 + at])[d & 7] = (_Float16)(v - (float)h);
-    };
+    float sn[kPairs], cs[kPairs];
+    int m_last = -1;
 #pragma unroll
-    for (int k = 0; k < kPairs; k++) {
-      const int i = tid + 64 * kTileWaves * k;
-      if (i >= n_pairs) break;
-      const int r = i / half, j = i - r * half;
-      float sn, cs;
-      sincosf(((float)(a.pos_base + (r0 + r) / a.G) / rp.pos_div) * qf[k], &sn, &cs);
-      put(r, j, (qa[k] * cs - qb[k] * sn) * a.qscale);
-      put(r, j + half, (qa[k] * sn + qb[k] * cs) * a.qscale);
+    for (int i = 0; i < kWaveRows; i++) {
+      const int r = wr0 + i;
+      if (i >= wave_rows || r >= nr) break;
+      const int m = wave_uniform((r0 + r) / a.G);
+      if (m != m_last) {
+#pragma unroll
+        for (int k = 0; k < kPairs; k++)
+          sincosf(((float)(a.pos_base + m) / rp.pos_div) * qf[k], &sn[k], &cs[k]);
+        m_last = m;
+      }
+      float mx = 0.f;
+#pragma unroll
+      for (int k = 0; k < kPairs; k++) {
+        const float x0 = qa[i][k], x1 = qb[i][k];
+        mx = fmaxf(mx, fmaxf(fabsf(x0), fabsf(x1)));
+        qa[i][k] = (x0 * cs[k] - x1 * sn[k]) * a.qscale;
+        qb[i][k] = (x0 * sn[k] + x1 * cs[k]) * a.qscale;
+      }
+      const int qe = exponent(attn::groups_max(max16(mx)) * a.qscale);
+      if (lane == 0) lds.qexp[r] = qe;
+#pragma unroll
+      for (int k = 0; k < kPairs; k++) {
+        const int j = lane + 64 * k;
+        if (j >= half) break;
+#pragma unroll
+        for (int b = 0; b < 2; b++) {
+          const int d = j + b * half, u = d >> 3;
+          const int at = (u >> 2) * 64 + (u & 3) * 16 + r;
+          float v = ldexpf(b ? qb[i][k] : qa[i][k], qe);
+#pragma unroll
+          for (int p = 0; p < Sh::QP; p++) {
+            asm("" : "+v"(v));
+            const _Float16 h = (_Float16)v;
+            reinterpret_cast<_Float16*>(&lds.qop[p * Sh::KS * 64 + at])[d & 7] = h;
+            v -= (float)h;
+          }
+        }
+      }
     }
   }
   __syncthreads();
+  const int unscale = -lds.qexp[l16];  // of this lane's row's logits
 
   // ---- the wave's tiles --------------------------------------------------
   const int lim = l16 < nr ? a.pos_base + (r0 + l16) / a.G : -1;
@@ -273,7 +360,7 @@ __global__ __launch_bounds__(64 * kTileWaves) void gen_tile_kernel(GenArgs a, Ge
     f4_t s[2] = {f4_t{0.f, 0.f, 0.f, 0.f}, f4_t{0.f, 0.f, 0.f, 0.f}};
     {
       struct Batch {
-        h8_t qh[2], ql[2];
+        h8_t q[2][Sh::QP];
         uint4 k[2][2];
       } cur, nxt;
       auto read = [&](int k0, Batch& f) {
@@ -281,8 +368,8 @@ __global__ __launch_bounds__(64 * kTileWaves) void gen_tile_kernel(GenArgs a, Ge
         for (int i = 0; i < 2; i++) {
           const int ks = k0 + i;
           if (ks >= Sh::KS) break;
-          f.qh[i] = lds.qop[ks * 64 + lane];
-          f.ql[i] = lds.qop[(Sh::KS + ks) * 64 + lane];
+#pragma unroll
+          for (int p = 0; p < Sh::QP; p++) f.q[i][p] = lds.qop[(p * Sh::KS + ks) * 64 + lane];
 #pragma unroll
           for (int tb = 0; tb < 2; tb++)
             f.k[i][tb] = *reinterpret_cast<const uint4*>(kst + tr.at(16 * tb + l16, 4 * ks + grp));
@@ -304,8 +391,11 @@ __global__ __launch_bounds__(64 * kTileWaves) void gen_tile_kernel(GenArgs a, Ge
             if (32 * ks + 32 > Sh::kLeast && 8 * (4 * ks + grp) >= dph)
               kx = make_uint4(0u, 0u, 0u, 0u);
             const h8_t k8 = __builtin_bit_cast(h8_t, kx);
-            s[tb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(k8, cur.qh[i], s[tb], 0, 0, 0);
-            s[tb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(k8, cur.ql[i], s[tb], 0, 0, 0);
+            // the smallest part first: fewer sums are rounded at the logit's
+            // magnitude (error at q x 16, head size 96: 2.0e-6 -> 1.2e-6)
+#pragma unroll
+            for (int p = Sh::QP - 1; p >= 0; p--)
+              s[tb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(k8, cur.q[i][p], s[tb], 0, 0, 0);
           }
         }
         cur = nxt;
@@ -336,7 +426,7 @@ __global__ __launch_bounds__(64 * kTileWaves) void gen_tile_kernel(GenArgs a, Ge
 #pragma unroll
       for (int i = 0; i < 4; i++) {
         const int pos = ts + 16 * tb + 4 * grp + i;
-        s[tb][i] = pos <= lim && pos < t1 ? s[tb][i] : kNegInf;
+        s[tb][i] = pos <= lim && pos < t1 ? ldexpf(s[tb][i], unscale) : kNegInf;
         mx = fmaxf(mx, s[tb][i]);
       }
     const float m_new = fmaxf(m_run, attn::groups_max(mx));

@@ -1,0 +1,65 @@
+"""The generic attention path's matrix-core form (gen_tile_kernel) over the
+range of inputs that its fp32 form takes, against float64.
+
+Queries of any finite magnitude: rows of a group that differ by a power of
+two of 40, at head sizes with two and with three fp16 parts of q, the
+smallest and the largest, with and without RoPE.
+
+Tolerance: a scaled row carries q to 2^-22 of its largest element and more, a
+logit's sum is fp32 and the logits here are N(0, 1) or smaller, so weights
+are within some 2^-20 relative and outputs within 1e-5 of their scale."""
+import numpy as np
+import pytest
+import torch
+
+from conftest import case_banner
+from speculative_decode_engine_amd import KVCache
+from speculative_decode_engine_amd import workloads as W
+
+pytestmark = pytest.mark.gpu
+
+
+def build(rng, K, V, nkv, dph, bs):
+    """A cache of one layer that holds the fp32 rows K, V behind a fragmented
+    table; returns it and the rows as fp16 stored them."""
+    n = -(-K.shape[0] // bs) + 1
+    cache = KVCache(1, nkv * dph, n, bs, n + 7)
+    cache.set_block_table(0, W.make_tables(rng, 1, n, n + 7)[0])
+    with np.errstate(over="ignore"):
+        K16, V16 = K.astype(np.float16), V.astype(np.float16)
+    cache.write_fp16(0, torch.from_numpy(K16.view(np.int16)).cuda(),
+                     torch.from_numpy(V16.view(np.int16)).cuda(), 0)
+    return cache, K16.astype(np.float32), V16.astype(np.float32)
+
+
+def rows(rng, n, width, scale=1.0):
+    return (rng.standard_normal((n, width)) * scale).astype(np.float32)
+
+
+@pytest.mark.parametrize("rope", [False, True])
+@pytest.mark.parametrize("qexp,kexp", [(20, -20), (-12, 10)])
+@pytest.mark.parametrize("nh,nkv,dph,bs", [(4, 2, 8, 16), (4, 2, 64, 12), (3, 1, 96, 16),
+                                           (8, 2, 256, 16)])
+def test_queries_of_any_magnitude(gpu, oracle, nh, nkv, dph, bs, qexp, kexp, rope):
+    case_banner("query range", nh, nkv, dph, bs, qexp, kexp, rope)
+    rng = np.random.default_rng(dph + qexp + 2 * rope + 12)
+    ctx, M = 300, 5
+    K, V = rows(rng, ctx + M, nkv * dph, 2.0 ** kexp), rows(rng, ctx + M, nkv * dph)
+    q = rows(rng, M, nh * dph, 2.0 ** qexp)
+    q[1] *= 2.0 ** -20
+    q[3] *= 2.0 ** -40
+    q[:, :dph // 2] *= 2.0 ** -6  # (a head whose elements differ)
+    cache, K, V = build(rng, K, V, nkv, dph, bs)
+    qt = torch.from_numpy(q).cuda()
+    if rope:
+        k, v = rows(rng, M, nkv * dph, 2.0 ** kexp), rows(rng, M, nkv * dph)
+        out = cache.rope_append_attention(0, qt, torch.from_numpy(k).cuda(),
+                                          torch.from_numpy(v).cuda(), nh, nkv, dph, ctx)
+        K, V = (t.cpu().numpy() for t in cache.read(0, 0, ctx + M))
+        q = oracle.rope_rotate_half_f64(q, nh, dph, np.arange(ctx, ctx + M))
+    else:
+        out = cache.attention(0, qt, nh, nkv, dph, ctx)
+    ref = oracle.attention_f64_np(q, K, V, nh, nkv, dph, ctx)
+    err = np.abs(out.cpu().numpy() - ref).max(axis=1) / np.abs(ref).max(axis=1)
+    assert (err <= 1e-5).all(), err
+    cache.free()
