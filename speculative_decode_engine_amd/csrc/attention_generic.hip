@@ -54,7 +54,7 @@ __global__ __launch_bounds__(kThreads) void gen_rope_append_kernel(GenArgs a, Ge
 //    in fp32 (the layouts of attention_device.hpp's tile path).  A row of q
 //    is scaled by a power of two into fp16's range first and its logits back
 //    (any finite q works, and a lo part never loses bits to fp16's least
-//    exponent);
+//    exponent), the weights by kWeightScale;
 //  * the waves' sums meet in LDS, the partitions' in a combine kernel.
 // Bound by the latency of a few tiles in turn and, as they grow, by memory.
 // Measured on MI355X, us per layer, fp32 form / this: decode over 3000 keys,
@@ -65,6 +65,13 @@ __global__ __launch_bounds__(kThreads) void gen_rope_append_kernel(GenArgs a, Ge
 // DPHP: the head size rounded up to a multiple of 32.
 constexpr int kTileWaves = 4;
 constexpr int kTileRows = 16;
+// The softmax weights, at most 1, enter the matrix cores times this (and
+// leave the sums exactly): fp16 then resolves 2^-40 of a row's largest weight
+// and not 2^-25, below which a key beside a dominant one was lost or rounded
+// to few bits (an attention sink 14 nats above the other keys, its V 0.02 of
+// theirs, 16/16 heads of 96, 1200 keys: error 1.2e-5, this 2.4e-7, the fp32
+// form 9e-7).
+constexpr float kWeightScale = 32768.f;
 
 using attn::f4_t;
 using attn::h8_t;
@@ -465,6 +472,8 @@ __global__ __launch_bounds__(64 * kTileWaves) void gen_tile_kernel(GenArgs a, Ge
       read(0, cur);
       __builtin_amdgcn_sched_barrier(0);
       h8_t ph, pl;
+#pragma unroll
+      for (int i = 0; i < 8; i++) p[i] *= kWeightScale;
       attn::split_h8(p, ph, pl);
 #pragma unroll
       for (int d0 = 0; d0 < Sh::DB; d0 += kBatch) {
@@ -489,7 +498,7 @@ __global__ __launch_bounds__(64 * kTileWaves) void gen_tile_kernel(GenArgs a, Ge
       for (int tb = 0; tb < 2; tb++)
 #pragma unroll
         for (int i = 0; i < 4; i++)
-          pt[l16 * attn::kTile + 16 * tb + 4 * grp + i] = p[4 * tb + i];
+          pt[l16 * attn::kTile + 16 * tb + 4 * grp + i] = p[4 * tb + i] * kWeightScale;
 #pragma unroll 1
       for (int t = 0; t < attn::kTile; t++) {
         const float w = pt[l16 * attn::kTile + t];
@@ -542,8 +551,8 @@ __global__ __launch_bounds__(64 * kTileWaves) void gen_tile_kernel(GenArgs a, Ge
       const float2 x = *reinterpret_cast<const float2*>(
           reinterpret_cast<const float*>(lds.st + w * Sh::WAVEB) + r * DPHP + d);
       l += ml[w].y * wt;
-      x0 += x.x * wt;
-      x1 += x.y * wt;
+      x0 += x.x * (wt * (1.f / kWeightScale));
+      x1 += x.y * (wt * (1.f / kWeightScale));
     }
     const int gr = r0 + r;
     if (a.n_parts == 1) {

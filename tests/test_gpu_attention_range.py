@@ -1,13 +1,5 @@
 """The generic attention path's matrix-core form (gen_tile_kernel) over the
-range of inputs that its fp32 form takes, against float64.
-
-Queries of any finite magnitude: rows of a group that differ by a power of
-two of 40, at head sizes with two and with three fp16 parts of q, the
-smallest and the largest, with and without RoPE.
-
-Tolerance: a scaled row carries q to 2^-22 of its largest element and more, a
-logit's sum is fp32 and the logits here are N(0, 1) or smaller, so weights
-are within some 2^-20 relative and outputs within 1e-5 of their scale."""
+range of inputs that its fp32 form takes, against float64."""
 import numpy as np
 import pytest
 import torch
@@ -41,6 +33,11 @@ def rows(rng, n, width, scale=1.0):
 @pytest.mark.parametrize("nh,nkv,dph,bs", [(4, 2, 8, 16), (4, 2, 64, 12), (3, 1, 96, 16),
                                            (8, 2, 256, 16)])
 def test_queries_of_any_magnitude(gpu, oracle, nh, nkv, dph, bs, qexp, kexp, rope):
+    """Rows of a group that differ by a power of two of 40, at head sizes with
+    two and with three fp16 parts of q, the smallest and the largest.  A scaled
+    row carries q to 2^-22 of its largest element, a logit's sum is fp32 and
+    the logits here are N(0, 1) or smaller, so weights are within some 2^-20
+    and outputs within 1e-5 of their scale."""
     case_banner("query range", nh, nkv, dph, bs, qexp, kexp, rope)
     rng = np.random.default_rng(dph + qexp + 2 * rope + 12)
     ctx, M = 300, 5
@@ -62,4 +59,36 @@ def test_queries_of_any_magnitude(gpu, oracle, nh, nkv, dph, bs, qexp, kexp, rop
     ref = oracle.attention_f64_np(q, K, V, nh, nkv, dph, ctx)
     err = np.abs(out.cpu().numpy() - ref).max(axis=1) / np.abs(ref).max(axis=1)
     assert (err <= 1e-5).all(), err
+    cache.free()
+
+
+@pytest.mark.parametrize("gap", [8.0, 14.0])
+@pytest.mark.parametrize("nh,nkv,dph,bs,ctx,M", [
+    (32, 32, 40, 16, 1200, 256),  # one partition: a wave's 300 keys beside the sink
+    (16, 8, 256, 16, 4000, 5),
+    (4, 2, 96, 16, 120, 1),       # a wave's 32 keys
+])
+def test_keys_beside_a_dominant_one(gpu, oracle, nh, nkv, dph, bs, ctx, M, gap):
+    """One key `gap` nats above the others whose V is small, as an attention
+    sink's: the other keys' weights of some e^-gap make a visible part of the
+    output.
+
+    A weight of 2^-20 of the largest is carried to 2^-22 and the rest of the
+    arithmetic is fp32: a logit near 25 (log2) is within some 2^-20, which its
+    key's weight takes on, and half the output (gap 8) or some percent of it
+    (gap 14) comes from the other keys' independent errors: 2e-6 in all."""
+    case_banner("dominant key", nh, nkv, dph, ctx, M, gap)
+    rng = np.random.default_rng(dph + int(gap))
+    u = np.sign(rng.standard_normal(dph)).astype(np.float32)
+    K, V = rows(rng, ctx + M, nkv * dph), rows(rng, ctx + M, nkv * dph)
+    K[0] = np.tile(u * np.float32(gap / np.sqrt(dph)), nkv)
+    V[0] *= 0.02
+    q = rows(rng, M, nh * dph) + np.tile(u, nh)
+    cache, K, V = build(rng, K, V, nkv, dph, bs)
+    out = cache.attention(0, torch.from_numpy(q).cuda(), nh, nkv, dph, ctx).cpu().numpy()
+    for m in range(0, M, max(1, M // 6)):
+        ref = oracle.attention_f64_np(q[m:m + 1], K[:ctx + m + 1], V[:ctx + m + 1], nh, nkv, dph,
+                                      ctx + m)
+        err = np.linalg.norm(out[m] - ref[0]) / np.linalg.norm(ref[0])
+        assert err <= 2e-6, (m, err)
     cache.free()
