@@ -54,7 +54,9 @@ struct GenArgs {
   const int32_t* table;
   const float* q;
   float* out;
-  float* partials;  // [nkv][R][n_parts][dph + 2]: acc, then max, sum
+  // [nkv][R][n_parts][dph + 2]: acc, then max, sum; or (gen_unit's PAIRS)
+  // [nkv][R][n_parts][dph], then (max, sum) pairs [nkv][R][n_parts]
+  float* partials;
   int kv_dim, bs;
   int nh, nkv, dph, G, R;
   int pos_base, L_max, n_parts, part_len;
@@ -101,8 +103,9 @@ struct GenLds {
 // Work unit (part, KV head h, row group rg) on the calling workgroup
 // (blockDim.x >= NT; every thread calls it): writes the normalised rows
 // (one partition) or their partial (acc, max, sum).  rp: the RoPE of q when
-// ROPE (k was rotated by the append).
-template <bool ROPE, int NT>
+// ROPE (k was rotated by the append).  PAIRS: the second layout of partials,
+// acc 0 where the row sees no key of the partition.
+template <bool ROPE, int NT, bool PAIRS = false>
 __device__ __forceinline__ void gen_unit(const GenArgs& a, const GenRope* rp, int part, int h,
                                          int rg, GenLds& lds) {
   static_assert(NT == 64 || NT == 128 || NT == 256, "active threads");
@@ -258,15 +261,18 @@ __device__ __forceinline__ void gen_unit(const GenArgs& a, const GenRope* rp, in
         if (d < dph) a.out[(size_t)m * a.nh * dph + (size_t)head * dph + d] = acc[r][k] * inv;
       }
     } else {
-      float* pp = a.partials + (((size_t)h * a.R + rho) * a.n_parts + part) * (size_t)(dph + 2);
+      const size_t pr = ((size_t)h * a.R + rho) * a.n_parts + part;
+      float* pp = a.partials + pr * (size_t)(PAIRS ? dph : dph + 2);
+      float* ml = PAIRS ? a.partials + (size_t)a.nkv * a.R * a.n_parts * dph + 2 * pr : pp + dph;
+      const bool none = PAIRS && row_l[r] == 0.f;
 #pragma unroll
       for (int k = 0; k < FPT; k++) {
         const int d = tid + NT * k;
-        if (d < dph) pp[d] = acc[r][k];
+        if (d < dph) pp[d] = none ? 0.f : acc[r][k];
       }
       if (tid == 0) {
-        pp[dph] = row_m[r];
-        pp[dph + 1] = row_l[r];
+        ml[0] = row_m[r];
+        ml[1] = row_l[r];
       }
     }
   }

@@ -99,10 +99,14 @@ struct TileLds {
   using Sh = TileShape<DPHP>;
   // (+ 1 KiB: a feature block past the head size is read, and dropped, from
   // behind the tile's last row)
-  char st[kTileWaves * Sh::WAVEB + 1024] __attribute__((aligned(16)));
+  union {
+    char st[kTileWaves * Sh::WAVEB + 1024] __attribute__((aligned(16)));
+    GenLds unit;
+  };
   h8_t qop[Sh::QP * Sh::KS * 64];
   int qexp[kTileRows];  // rows of q: the exponent of the power of two on it
   float2 ml[kTileWaves][kTileRows];
+  int nonfinite[kTileWaves];
   static_assert(kTileRows * DPHP * 4 <= Sh::WAVEB, "a wave's sums fit its tiles");
 };
 
@@ -535,6 +539,7 @@ __global__ __launch_bounds__(64 * kTileWaves) void gen_tile_kernel(GenArgs a, Ge
   // ---- the waves' sums meet: thread -> (row, 2 features) ---------------
   const size_t n_acc = (size_t)a.nkv * a.R * a.n_parts * dph;  // then (max, sum) pairs
   const int hp = dph / 2;
+  float finite = 0.f;  // NaN where a sum is not finite
   for (int i = tid; i < nr * hp; i += 64 * kTileWaves) {
     const int r = i / hp, d = 2 * (i - r * hp);
     float2 ml[kTileWaves];
@@ -554,6 +559,7 @@ __global__ __launch_bounds__(64 * kTileWaves) void gen_tile_kernel(GenArgs a, Ge
       x0 += x.x * (wt * (1.f / kWeightScale));
       x1 += x.y * (wt * (1.f / kWeightScale));
     }
+    finite = fmaf(l, 0.f, fmaf(x0, 0.f, fmaf(x1, 0.f, finite)));
     const int gr = r0 + r;
     if (a.n_parts == 1) {
       const int m = gr / a.G, h = kvh * a.G + (gr - m * a.G);
@@ -565,6 +571,22 @@ __global__ __launch_bounds__(64 * kTileWaves) void gen_tile_kernel(GenArgs a, Ge
       *reinterpret_cast<float2*>(a.partials + pr * dph + d) = make_float2(x0, x1);
       if (d == 0) *reinterpret_cast<float2*>(a.partials + n_acc + pr * 2) = make_float2(mx, l);
     }
+  }
+
+  // A part of a pair can make NaN (Inf x 0, Inf - Inf) of a product with Inf
+  // that is Inf, or weighs nothing, in fp32: where a row's sums are not finite
+  // the fp32 work unit does the partition's rows over, after these stores.
+  // (The test costs 0.1 us of a layer's 20 at 32 heads of 96.)
+  const bool nonfinite = __builtin_amdgcn_ballot_w64(finite != finite) != 0;
+  if (lane == 0) lds.nonfinite[wave] = nonfinite;
+  __syncthreads();
+  if ((lds.nonfinite[0] | lds.nonfinite[1] | lds.nonfinite[2] | lds.nonfinite[3]) == 0) return;
+  __builtin_amdgcn_s_waitcnt(0);
+  for (int g = rg * (kTileRows / kGenRows); g * kGenRows < r0 + nr; g++) {
+    if (use_rope)
+      gen_unit<true, 64 * kTileWaves, true>(a, &rp, part, kvh, g, lds.unit);
+    else
+      gen_unit<false, 64 * kTileWaves, true>(a, &rp, part, kvh, g, lds.unit);
   }
 }
 

@@ -92,3 +92,54 @@ def test_keys_beside_a_dominant_one(gpu, oracle, nh, nkv, dph, bs, ctx, M, gap):
         err = np.linalg.norm(out[m] - ref[0]) / np.linalg.norm(ref[0])
         assert err <= 2e-6, (m, err)
     cache.free()
+
+
+def special(x):
+    """0 where finite, 1 / -1 where +-Inf, 2 where NaN."""
+    return np.where(np.isnan(x), 2, np.where(np.isinf(x), np.sign(x), 0))
+
+
+@pytest.mark.parametrize("rope", [False, True])
+@pytest.mark.parametrize("what", ["V", "K", "q"])
+@pytest.mark.parametrize("nh,nkv,dph,bs,ctx,M", [
+    (4, 2, 32, 16, 300, 3),      # three partitions
+    (4, 2, 96, 16, 100, 1),      # one partition
+    (10, 2, 256, 12, 700, 5),    # 25 rows: two groups of rows
+    (4, 4, 40, 16, 900, 21),
+])
+def test_nonfinite_values_that_rows_see(gpu, oracle, nh, nkv, dph, bs, ctx, M, what, rope):
+    """Inf in V reaches its features with its sign, a logit of -Inf weighs
+    nothing and one of +Inf or NaN makes its row NaN, as fp32 arithmetic has
+    it; every other output keeps its precision."""
+    case_banner("visible non-finite", nh, nkv, dph, bs, ctx, M, what, rope)
+    rng = np.random.default_rng(dph + ctx)
+    K, V = rows(rng, ctx + M, nkv * dph), rows(rng, ctx + M, nkv * dph)
+    q = rows(rng, M, nh * dph)
+    if what == "V":
+        V[7, ::3], V[90, 1::3] = np.inf, -np.inf
+        V[40, dph - 1] = np.nan
+    elif what == "K":
+        K[70, 3] = np.inf
+        q.reshape(M, nh, dph)[:, ::2, 3] = -1.0
+    else:
+        q[0, 5], q[M - 1, dph + 2] = np.inf, np.nan
+    cache, K, V = build(rng, K, V, nkv, dph, bs)
+    qt = torch.from_numpy(q).cuda()
+    if rope:
+        k, v = rows(rng, M, nkv * dph), rows(rng, M, nkv * dph)
+        out = cache.rope_append_attention(0, qt, torch.from_numpy(k).cuda(),
+                                          torch.from_numpy(v).cuda(), nh, nkv, dph, ctx)
+        K, V = (t.cpu().numpy() for t in cache.read(0, 0, ctx + M))
+        with np.errstate(invalid="ignore"):
+            q = oracle.rope_rotate_half_f64(q, nh, dph, np.arange(ctx, ctx + M))
+    else:
+        out = cache.attention(0, qt, nh, nkv, dph, ctx)
+    with np.errstate(invalid="ignore", over="ignore"):
+        ref = oracle.attention_f64_np(q, K, V, nh, nkv, dph, ctx)
+    got = out.cpu().numpy()
+    # (RoPE gives the feature that meets K's Inf either sign)
+    assert (special(ref) == 0).any() and (what == "K" or (special(ref) != 0).any())
+    assert np.array_equal(special(got), special(ref)), np.argwhere(special(got) != special(ref))[:8]
+    live = special(ref) == 0
+    assert np.abs(got[live] - ref[live]).max() <= 1e-5 * np.abs(ref[live]).max()
+    cache.free()
