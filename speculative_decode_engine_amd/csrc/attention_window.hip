@@ -19,8 +19,8 @@
 //    past a wave's are not multiplied;
 //  * the weights' reference (the running max) enters the logits product as
 //    its initial accumulator and is raised only when a row's max is more
-//    than 2^8 above it (weights up to 2^8 are as exact in fp16 hi + lo),
-//    which skips most rescales of the output registers.
+//    than 2^8 above it, which skips most rescales of the output registers;
+//    the weights enter the products times 2^7 (kWeightScale), below 2^15.
 // Tiles go from memory straight into LDS, one ahead of the one multiplied
 // (two buffers, one barrier per tile): carried in registers instead, the
 // next tile's 16-32 registers made the kernel spill, and its loads, 2 us
@@ -52,6 +52,13 @@ constexpr int kHalf = 32;       // tokens of a tile that one wave takes
 constexpr int kWinBuffers = 2;  // tiles in LDS: one multiplied, one on its way
 constexpr int kWinTable = 2048; // block table entries in LDS
 constexpr float kLazyMax = 8.f;  // log2 growth of a row's max that triggers a rescale
+// On the weights (up to 2^kLazyMax) where they enter the matrix cores, taken
+// back from the sums exactly: fp16's quantum is then 2^-32 of the reference
+// and not 2^-25, which a key beside a dominant one is rounded to.  One
+// reference spans a row's partition here, where the 16-row kernels have one
+// per wave (a sink 14 nats above the other keys, its V 0.02 of theirs, 2003
+// keys, 32/8 heads of 128: error 2.0e-5, this 3.7e-7, 16-row kernel 1.0e-5).
+constexpr float kWeightScale = 128.f;
 
 template <int DPH>
 struct WinShape {
@@ -144,7 +151,7 @@ __device__ __forceinline__ void win_exact_pv(int ts, int lane, int lim, const f1
   for (int c = 0; c < 32 / CT; c++) {
     // tokens 8c .. 8c+7: registers 4c .. 4c+3 of both halves
 #pragma unroll
-    for (int i = 0; i < 4; i++) pt[l32 * CT + 4 * hf + i] = s[4 * c + i];
+    for (int i = 0; i < 4; i++) pt[l32 * CT + 4 * hf + i] = s[4 * c + i] * kWeightScale;
 #pragma unroll 1
     for (int t = 0; t < CT; t++) {
       const float w = pt[l32 * CT + t];
@@ -466,7 +473,7 @@ __global__ __launch_bounds__(kWinThreads) void attn_window_kernel(AttnArgs a) {
       for (int k2 = 0; k2 < 2; k2++) {
         float x[8];
 #pragma unroll
-        for (int i = 0; i < 8; i++) x[i] = s[8 * k2 + i];
+        for (int i = 0; i < 8; i++) x[i] = s[8 * k2 + i] * kWeightScale;
         split_weights(x, ph[k2], pl[k2]);
       }
       read_v(1);
@@ -527,12 +534,13 @@ __global__ __launch_bounds__(kWinThreads) void attn_window_kernel(AttnArgs a) {
     const float wa1 = sums_weight(y.x, y.y, m);
     m_row = m;
     l_row = l_row * wa0 + y.y * wa1;
+    const float wo0 = wa0 * (1.f / kWeightScale), wo1 = wa1 * (1.f / kWeightScale);
 #pragma unroll
     for (int i = 0; i < 4 * Sh::DB; i++) {
       const f4_t x = xo[64 * i];
 #pragma unroll
       for (int e = 0; e < 4; e++)
-        o[i / 4][4 * (i & 3) + e] = o[i / 4][4 * (i & 3) + e] * wa0 + x[e] * wa1;
+        o[i / 4][4 * (i & 3) + e] = o[i / 4][4 * (i & 3) + e] * wo0 + x[e] * wo1;
     }
   }
   const int m = row / a.G;

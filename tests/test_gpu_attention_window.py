@@ -70,6 +70,36 @@ def test_wide_window_matches_float64(gpu, oracle, nh, nkv, dph, bs, ctx, M):
     cache.free()
 
 
+@pytest.mark.parametrize("nh,nkv,dph,ctx,M,gap", [
+    (32, 8, 128, 0, 2003, 14.0),
+    (32, 8, 128, 0, 2003, 8.0),
+    (32, 4, 64, 1500, 256, 14.0),   # partitions
+])
+def test_keys_beside_a_dominant_one(gpu, oracle, nh, nkv, dph, ctx, M, gap):
+    """One key `gap` nats above the others whose V is small, as an attention
+    sink's: the other keys' weights of some e^-gap make a visible part of the
+    output.
+
+    A weight of 2^-20 of the largest is carried to 2^-12 of itself at the
+    least (a quantum of 2^-32) and the rest of the arithmetic is fp32; half the
+    output (gap 8) or some percent of it (gap 14) comes from the other keys,
+    whose errors are independent: 2e-6 in all."""
+    case_banner("wide window, dominant key", nh, nkv, dph, ctx, M, gap)
+    cache, K, V, rng = build_layer(nh, nkv, dph, 16, ctx, M, -(-(ctx + M) // 16) + 7, dph + M)
+    u = np.sign(rng.standard_normal(dph)).astype(np.float32)
+    K[0] = np.tile(u * np.float32(gap / np.sqrt(dph)), nkv).astype(np.float16)
+    V[0] = (V[0] * 0.02).astype(np.float16)
+    cache.append(0, torch.from_numpy(K[:1].copy()).cuda(), torch.from_numpy(V[:1].copy()).cuda(), 0)
+    q = W.queries(rng, M, nh, dph) + np.tile(u, nh)
+    out = cache.attention(0, torch.from_numpy(q).cuda(), nh, nkv, dph, ctx).cpu().numpy()
+    for m in sorted({M // 2, M - 1} | set(range(M // 3, M, max(1, M // 8)))):
+        ref = oracle.attention_f64_np(q[m:m + 1], K[:ctx + m + 1], V[:ctx + m + 1], nh, nkv, dph,
+                                      ctx + m)
+        err = np.linalg.norm(out[m] - ref[0]) / np.linalg.norm(ref[0])
+        assert err <= 2e-6, (m, err)
+    cache.free()
+
+
 @pytest.mark.parametrize("dph", [64, 128])
 def test_wide_window_hidden_nonfinite_rows(gpu, oracle, dph):
     """Inf / NaN in V (and NaN in K) at window positions and in stale slots
