@@ -164,8 +164,8 @@ size_t pool_bytes_of(const sde_kv_config& c) {
 void release(sde_kv_cache* c) {
   if (!c) return;
   if (c->owns_pool && c->pool) (void)hipFree(c->pool);
-  if (c->workspace && c->workspace != c->arena) (void)hipFree(c->workspace);
   if (c->arena) (void)hipFree(c->arena);
+  if (c->workspace) (void)hipFree(c->workspace);
   for (void* w : c->retired_workspaces) (void)hipFree(w);
   delete c;
 }
@@ -185,26 +185,18 @@ int finish_create(sde_kv_cache* c, sde_kv_cache** out) {
       c->n_mapped[l] = cfg.max_blocks_per_layer;
     }
   }
-  // One allocation: the attention workspace (for caches of more than one
-  // partition's 256 keys: a call that has to allocate it takes 20 us and more
-  // longer; larger plans still grow it), the tables, the counters (zero at
-  // rest) and seq_len.
-  const size_t ws = (int64_t)cfg.max_blocks_per_layer * cfg.block_size > 256
-                        ? sde::kInitialWorkspace
-                        : 0;
+  // One allocation: the tables, the counters (zero at rest) and seq_len.
   const size_t tables = (n_entries * sizeof(int32_t) + 255) / 256 * 256;
   const size_t counters =
       ((size_t)sde::kMaxAttnCounters + sde::kSpecScratchWords) * sizeof(uint32_t);
-  if (hipMalloc(&c->arena, ws + tables + counters + sizeof(int32_t)) != hipSuccess) {
+  if (hipMalloc(&c->arena, tables + counters + sizeof(int32_t)) != hipSuccess) {
     release(c);
     return SDE_ERR_HIP;
   }
   char* base = static_cast<char*>(c->arena);
-  c->workspace = ws > 0 ? base : nullptr;
-  c->workspace_bytes = ws;
-  c->d_tables = reinterpret_cast<int32_t*>(base + ws);
-  c->d_counters = reinterpret_cast<uint32_t*>(base + ws + tables);
-  c->d_seq_len = reinterpret_cast<int32_t*>(base + ws + tables + counters);
+  c->d_tables = reinterpret_cast<int32_t*>(base);
+  c->d_counters = reinterpret_cast<uint32_t*>(base + tables);
+  c->d_seq_len = reinterpret_cast<int32_t*>(base + tables + counters);
   if (hipMemcpy(c->d_tables, c->h_tables.data(), n_entries * sizeof(int32_t),
                 hipMemcpyHostToDevice) != hipSuccess ||
       hipMemset(c->d_counters, 0, counters + sizeof(int32_t)) != hipSuccess ||

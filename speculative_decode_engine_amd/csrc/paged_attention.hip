@@ -196,18 +196,18 @@ bool serves_window(const sde_kv_cache* cache, int dph, int L_max, int nkv, int R
 
 // Lowers *most, the partials a plan may have, to what the call's workspace
 // holds: the caller's, or under stream capture (no allocation can be
-// recorded) what earlier calls took of the cache's.  SDE_ERR_WORKSPACE where
+// recorded) what earlier calls made the cache's.  SDE_ERR_WORKSPACE where
 // that is less than `need`.
 int workspace_limit(const sde_kv_cache* cache, size_t need, const void* d_workspace,
                     size_t workspace_bytes, sde_stream_t stream, size_t* most) {
   size_t have = *most;
   if (d_workspace) {
     have = workspace_bytes;
-  } else if (cache->workspace_used < *most) {
+  } else if (cache->workspace_bytes < *most) {
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing((hipStream_t)stream, &cap) != hipSuccess) return SDE_ERR_HIP;
     if (cap == hipStreamCaptureStatusNone) return SDE_OK;
-    have = cache->workspace_used;
+    have = cache->workspace_bytes;
   }
   if (have < need) return SDE_ERR_WORKSPACE;
   if (have < *most) *most = have;
@@ -266,27 +266,26 @@ int run_attention(sde_kv_cache* cache, int layer, const float* d_q, float* d_out
       if (workspace_bytes < need) return SDE_ERR_WORKSPACE;
       partials = static_cast<float*>(d_workspace);
     } else {
-      if (cache->workspace_used < need) {
-        // Take more of the cache-owned workspace, growing it where what was
-        // allocated at creation does not do.  Not while the stream is being
-        // captured: an allocation cannot be recorded, and a graph would
+      if (cache->workspace_bytes < need) {
+        // Grow the cache-owned workspace.  Not while the stream is being
+        // captured: the allocation cannot be recorded, and a graph would
         // keep its address.  The old buffer stays allocated (queued work
         // or an earlier graph may still use it) until the cache is freed,
-        // so the size at least doubles: a context that grows call by call
-        // retires O(log) buffers, at most about twice the peak need in all.
+        // so the size at least doubles, up to the most that any plan takes:
+        // a context that grows call by call retires O(log) buffers, at most
+        // about twice the peak need in all.
         hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
         if (hipStreamIsCapturing((hipStream_t)stream, &cap) != hipSuccess) return SDE_ERR_HIP;
         if (cap != hipStreamCaptureStatusNone) return SDE_ERR_WORKSPACE;
-        const size_t used = need > 2 * cache->workspace_used ? need : 2 * cache->workspace_used;
-        if (cache->workspace_bytes < used) {
-          void* grown = nullptr;
-          if (hipMalloc(&grown, used) != hipSuccess) return SDE_ERR_HIP;
-          if (cache->workspace && cache->workspace != cache->arena)
-            cache->retired_workspaces.push_back(cache->workspace);
-          cache->workspace = grown;
-          cache->workspace_bytes = used;
-        }
-        cache->workspace_used = used;
+        constexpr size_t kMost = SDE_NOALLOC_WIDE_SCRATCH_BYTES;
+        const size_t twice = 2 * cache->workspace_bytes;
+        const size_t ahead = twice < kMost ? twice : kMost;
+        const size_t grow = need > ahead ? need : ahead;
+        void* grown = nullptr;
+        if (hipMalloc(&grown, grow) != hipSuccess) return SDE_ERR_HIP;
+        if (cache->workspace) cache->retired_workspaces.push_back(cache->workspace);
+        cache->workspace = grown;
+        cache->workspace_bytes = grow;
       }
       partials = static_cast<float*>(cache->workspace);
     }

@@ -19,19 +19,15 @@ struct sde_kv_cache {
   uint16_t* pool = nullptr;
   size_t pool_bytes = 0;
   bool owns_pool = false;
-  void* arena = nullptr;                // workspace, tables, counters, seq_len
+  void* arena = nullptr;                // tables, counters, seq_len
   int32_t* d_tables = nullptr;          // [n_layers][max_blocks_per_layer]
   std::vector<int32_t> h_tables;        // host mirror of d_tables
   std::vector<int32_t> n_mapped;        // leading mapped logical blocks per layer
   int32_t* d_seq_len = nullptr;
   int seq_len = 0;                      // host mirror of *d_seq_len
   bool seq_len_on_device = false;       // *d_seq_len was set by a device-side rewind
-  void* workspace = nullptr;            // internal attention workspace
+  void* workspace = nullptr;            // internal attention workspace, grown on demand
   size_t workspace_bytes = 0;
-  // The part of it that calls so far have asked for (at least doubling): a
-  // call under stream capture, which must not be the first to need its size,
-  // is held against this and not against what was allocated ahead.
-  size_t workspace_used = 0;
   // Workspaces outgrown by a larger call: kept until the cache is
   // destroyed, because work already queued, or a graph captured earlier,
   // may still use them.
@@ -48,9 +44,6 @@ namespace sde {
 // acceptance's scratch (kSpecScratchWords, sde/spec_device.hpp: arrival
 // counters zero at rest, per-row results and per-slice statistics).
 constexpr int kMaxAttnCounters = 4096;
-// Bytes of a cache's attention workspace from its creation on: every plan's
-// partials (the wide windows' are the most, SDE_NOALLOC_WIDE_SCRATCH_BYTES).
-constexpr size_t kInitialWorkspace = SDE_NOALLOC_WIDE_SCRATCH_BYTES;
 }  // namespace sde
 
 namespace sde {
