@@ -29,6 +29,7 @@
 #include <atomic>
 #include <climits>
 #include <cmath>
+#include <cstdint>
 #include <cstdlib>
 #include <cstring>
 #include <mutex>
@@ -194,26 +195,6 @@ bool serves_window(const sde_kv_cache* cache, int dph, int L_max, int nkv, int R
          sde::win::window_serves(L_max, nkv, R);
 }
 
-// Lowers *most, the partials a plan may have, to what the call's workspace
-// holds: the caller's, or under stream capture (no allocation can be
-// recorded) what earlier calls made the cache's.  SDE_ERR_WORKSPACE where
-// that is less than `need`.
-int workspace_limit(const sde_kv_cache* cache, size_t need, const void* d_workspace,
-                    size_t workspace_bytes, sde_stream_t stream, size_t* most) {
-  size_t have = *most;
-  if (d_workspace) {
-    have = workspace_bytes;
-  } else if (cache->workspace_bytes < *most) {
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing((hipStream_t)stream, &cap) != hipSuccess) return SDE_ERR_HIP;
-    if (cap == hipStreamCaptureStatusNone) return SDE_OK;
-    have = cache->workspace_bytes;
-  }
-  if (have < need) return SDE_ERR_WORKSPACE;
-  if (have < *most) *most = have;
-  return SDE_OK;
-}
-
 int run_attention(sde_kv_cache* cache, int layer, const float* d_q, float* d_out, int nh,
                   int nkv, int dph, int pos_base, int n_queries, void* d_workspace,
                   size_t workspace_bytes, sde_stream_t stream, const RopeArgs* rope,
@@ -225,71 +206,79 @@ int run_attention(sde_kv_cache* cache, int layer, const float* d_q, float* d_out
   const int R = n_queries * G;
   const int L_max = pos_base + n_queries;
   const bool generic = sde::gen::needs_generic(dph, cache->cfg.block_size);
+  const bool tiles = generic && sde::gen::tile_serves(dph, cache->cfg.block_size,
+                                                      cache->cfg.pool_blocks);
+  const bool wide = !rope && serves_window(cache, dph, L_max, nkv, R);
   StreamPlan plan{};
   sde::gen::GenPlan gplan{};
   sde::win::WindowPlan wplan{};
-  size_t need = 0;
-  bool tiles = false;
+  size_t base = 0;  // bytes of the 16-row kernels' or the fp32 form's partials
   if (generic) {
     gplan = sde::gen::generic_plan(L_max, nkv, R, dph, cache->n_cus, parts_bound(L_max));
-    need = sde::gen::generic_partial_bytes(gplan, nkv, R, dph);
-    tiles = sde::gen::tile_serves(dph, cache->cfg.block_size, cache->cfg.pool_blocks);
-    if (tiles) {
-      // The matrix-core form has a plan of its own; its partials take what
-      // the workspace holds, and a call is refused for its workspace only
-      // where the fp32 form's plan is.
-      size_t most = SDE_NOALLOC_SCRATCH_BYTES;
-      const int st = workspace_limit(cache, need, d_workspace, workspace_bytes, stream, &most);
-      if (st != SDE_OK) return st;
-      gplan = sde::gen::tile_plan(L_max, nkv, R, dph, cache->n_cus, tile_parts_bound(L_max), most);
-      need = sde::gen::generic_partial_bytes(gplan, nkv, R, dph);
-    }
+    base = sde::gen::generic_partial_bytes(gplan, nkv, R, dph);
   } else {
     plan = plan_for(L_max, nkv, R, cache->n_cus);
     if ((int64_t)nkv * plan.row_groups > sde::kMaxAttnCounters) return SDE_ERR_UNSUPPORTED;
-    need = partial_bytes(nkv, R, plan.n_parts, dph);
+    base = partial_bytes(nkv, R, plan.n_parts, dph);
   }
-  const bool wide = !rope && serves_window(cache, dph, L_max, nkv, R);
-  if (wide) {
-    // A wide window: its own kernel and split.  Its partials take what the
-    // workspace holds (down to one partition, which needs none), and a call
-    // is refused for its workspace only where the 16-row kernels' plan is.
-    size_t most = SDE_NOALLOC_WIDE_SCRATCH_BYTES;
-    const int st = workspace_limit(cache, need, d_workspace, workspace_bytes, stream, &most);
-    if (st != SDE_OK) return st;
-    wplan = sde::win::window_plan(L_max, nkv, R, dph, cache->n_cus, parts_bound(L_max), most);
-    need = sde::win::window_partial_bytes(wplan, nkv, R, dph);
-  }
-  float* partials = nullptr;
-  if (need > 0) {
-    if (d_workspace) {
-      if (workspace_bytes < need) return SDE_ERR_WORKSPACE;
-      partials = static_cast<float*>(d_workspace);
+  // The matrix-core form and the wide windows have plans of their own, whose
+  // partials take what a workspace holds (down to one partition, which needs
+  // none).  A call is refused for its workspace only where the base plan is.
+  auto own_plan = [&](size_t most) {
+    if (tiles) {
+      if (most > SDE_NOALLOC_SCRATCH_BYTES) most = SDE_NOALLOC_SCRATCH_BYTES;
+      gplan = sde::gen::tile_plan(L_max, nkv, R, dph, cache->n_cus, tile_parts_bound(L_max), most);
+      return sde::gen::generic_partial_bytes(gplan, nkv, R, dph);
+    }
+    if (wide) {
+      if (most > SDE_NOALLOC_WIDE_SCRATCH_BYTES) most = SDE_NOALLOC_WIDE_SCRATCH_BYTES;
+      wplan = sde::win::window_plan(L_max, nkv, R, dph, cache->n_cus, parts_bound(L_max), most);
+      return sde::win::window_partial_bytes(wplan, nkv, R, dph);
+    }
+    return base;
+  };
+  size_t need = own_plan(d_workspace ? workspace_bytes : SIZE_MAX);
+  void* ws = d_workspace;
+  if (d_workspace) {
+    if (workspace_bytes < base || workspace_bytes < need) return SDE_ERR_WORKSPACE;
+  } else {
+    // The cache's own: room for both plans, so that the same call under
+    // stream capture finds all it takes and runs the same plan.  Not grown
+    // while the stream is being captured: the allocation cannot be recorded,
+    // and a graph would keep its address.  The old buffer stays allocated
+    // (queued work or an earlier graph may still use it) until the cache is
+    // freed, so the size at least doubles, up to the most that any plan
+    // takes: a context that grows call by call retires O(log) buffers, at most
+    // about twice the peak need in all.
+    size_t room = cache->workspace_base;
+    if (base > room) room = base > 2 * room ? base : 2 * room;
+    const size_t want = need > room ? need : room;
+    bool captured = false;
+    if (cache->workspace_bytes < want) {
+      hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+      if (hipStreamIsCapturing((hipStream_t)stream, &cap) != hipSuccess) return SDE_ERR_HIP;
+      captured = cap != hipStreamCaptureStatusNone;
+    }
+    if (captured) {
+      if (cache->workspace_bytes < base) return SDE_ERR_WORKSPACE;
+      need = own_plan(cache->workspace_bytes);
     } else {
-      if (cache->workspace_bytes < need) {
-        // Grow the cache-owned workspace.  Not while the stream is being
-        // captured: the allocation cannot be recorded, and a graph would
-        // keep its address.  The old buffer stays allocated (queued work
-        // or an earlier graph may still use it) until the cache is freed,
-        // so the size at least doubles, up to the most that any plan takes:
-        // a context that grows call by call retires O(log) buffers, at most
-        // about twice the peak need in all.
-        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-        if (hipStreamIsCapturing((hipStream_t)stream, &cap) != hipSuccess) return SDE_ERR_HIP;
-        if (cap != hipStreamCaptureStatusNone) return SDE_ERR_WORKSPACE;
+      if (cache->workspace_bytes < want) {
         constexpr size_t kMost = SDE_NOALLOC_WIDE_SCRATCH_BYTES;
         const size_t twice = 2 * cache->workspace_bytes;
-        const size_t ahead = twice < kMost ? twice : kMost;
-        const size_t grow = need > ahead ? need : ahead;
+        size_t grow = twice < kMost ? twice : kMost;
+        if (grow < want) grow = want;
         void* grown = nullptr;
         if (hipMalloc(&grown, grow) != hipSuccess) return SDE_ERR_HIP;
         if (cache->workspace) cache->retired_workspaces.push_back(cache->workspace);
         cache->workspace = grown;
         cache->workspace_bytes = grow;
       }
-      partials = static_cast<float*>(cache->workspace);
+      cache->workspace_base = room;
     }
+    ws = cache->workspace;
   }
+  float* const partials = need > 0 ? static_cast<float*>(ws) : nullptr;
 
   if (generic)
     return sde::gen::generic_attention(cache->pool, sde::layer_table(cache, layer),

@@ -28,6 +28,9 @@ struct sde_kv_cache {
   bool seq_len_on_device = false;       // *d_seq_len was set by a device-side rewind
   void* workspace = nullptr;            // internal attention workspace, grown on demand
   size_t workspace_bytes = 0;
+  // What the 16-row and fp32 plans of the calls so far take of it, at least
+  // doubled as it grows: never more than workspace_bytes.
+  size_t workspace_base = 0;
   // Workspaces outgrown by a larger call: kept until the cache is
   // destroyed, because work already queued, or a graph captured earlier,
   // may still use them.
