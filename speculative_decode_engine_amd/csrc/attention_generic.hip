@@ -418,6 +418,9 @@ __global__ __launch_bounds__(64 * kTileWaves) void gen_tile_kernel(GenArgs a, Ge
     asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory");
     // a tile that reaches a position some row may not see: non-finite V at
     // such a position must not meet its zero weight in the matrix product
+    // (such a tile is the wave's last: the rows' last positions differ by
+    // less than kTileRows, and the wave's next tile lies kStride further)
+    static_assert(kStride >= kTileRows + attn::kTile, "no tile after an exact one");
     bool exact = false;
     if (ts + attn::kTile - 1 > wmin) {
       uint32_t bad = 0;
@@ -430,7 +433,7 @@ __global__ __launch_bounds__(64 * kTileWaves) void gen_tile_kernel(GenArgs a, Ge
         }
       exact = __builtin_amdgcn_ballot_w64(bad != 0) != 0;
     }
-    if (more && !exact) load(row, k_off);
+    if (more) load(row, k_off);
     float mx = kNegInf;
 #pragma unroll
     for (int tb = 0; tb < 2; tb++)
@@ -522,7 +525,6 @@ __global__ __launch_bounds__(64 * kTileWaves) void gen_tile_kernel(GenArgs a, Ge
     __builtin_amdgcn_sched_barrier(0);
     asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory");  // the V tile is free
     if (more) {
-      if (exact) load(row, k_off);
       if (ts + 2 * kStride < t1) row_n = row_of(ts + 2 * kStride);
       load(row + (uint32_t)a.bs, k_off + Sh::TILEB);
     }
