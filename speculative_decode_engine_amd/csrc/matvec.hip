@@ -45,14 +45,16 @@ namespace mvp {
 // multiply-adds overlap more of the streaming (measured on MI355X, 5 rows
 // of the 14336 x 4096 W_down: 24.2 vs 25.2 us) and whose doubled step
 // registers stay within 256 VGPRs up to 9 rows.
-// Up to five rows within 128 VGPRs (five took 129), for two workgroups per
-// CU: a panel of few rows is read in four steps per wave, and a workgroup
-// alone on its CU streams nothing while it starts and while it sums (5 rows
-// of a 4096 x 128256 head 243 -> 186 us, of 2048 x 32000 41.3 -> 31.6, of
-// 4096 x 14336 33.1 -> 26.9; 4096 x 4096, one workgroup per CU, 10.5 / 10.2).
-// Six would need steps of two units, which cost 14336 x 4096 26.0 -> 32.1 us.
+// Five rows within 128 VGPRs (they took 129), for two workgroups per CU, as
+// fewer rows have by themselves (held to 128, three rows of 2048 x 32000 were
+// scheduled otherwise: 25.1 -> 25.8 us): a panel of few rows is read in four
+// steps per wave, and a workgroup alone on its CU streams nothing while it
+// starts and while it sums (5 rows of a 4096 x 128256 head 243 -> 187 us, of
+// 2048 x 32000 40.6 -> 31.3, of 4096 x 14336 32.8 -> 27.0; 4096 x 4096, one
+// workgroup per CU, 10.2 / 10.2).  Six would need steps of two units, which
+// cost 14336 x 4096 26.0 -> 32.1 us.
 template <int MB, int LPR>
-__global__ __launch_bounds__(64 * kWaves, MB <= 5 ? 4 : 2) void matvec_packed_kernel(PackedArgs a) {
+__global__ __launch_bounds__(64 * kWaves, MB == 5 ? 4 : 2) void matvec_packed_kernel(PackedArgs a) {
   packed_item<MB, LPR, (MB == 1 ? 8 : 4)>(a, blockIdx.x, blockIdx.y);
 }
 
