@@ -631,15 +631,25 @@ __global__ __launch_bounds__(256) void window_combine_kernel(AttnArgs a) {
 
 // The 16-row kernels spread a window over the chip in one round as long as
 // its rows and keys are few, and start faster (this kernel's first tile is
-// some 4 us away); their cost then grows with every 16 rows re-reading the
-// keys.  Measured on MI355X, us per call, 16-row kernels / this one, by rows
-// x keys over all KV heads: 32/8 heads of 128, 48 queries after 4000 keys
-// (6.2M) 28.5 / 29.0, 128 after 4000 (17M) 44 / 38, 512 after 4000 (74M)
-// 195 / 87, 24 after 16000 (12M) 49 / 37; 32/4 heads of 64, 24 after 16000
-// (12M) 28.0 / 27.7, 64 after 4000 (8.4M) 19 / 22, 128 after 4000 (17M)
-// 27.4 / 27.3; 8/8 heads of 128, 128 after 16000 (17M) 51 / 39.  From 16384
-// rows on the grid is half full without a split: 512 queries alone (8.4M)
-// 45 / 31 and 26 / 20.
+// some 4 us away); their cost then grows by rounds, and with every 16 rows
+// re-reading the keys.  Measured on MI355X, us per call, 16-row kernels /
+// this one, by rows x keys over all KV heads:
+//   32/8 heads of 128: 48 queries after 4000 keys (6M) 27.3 / 28.6, 64 (8M)
+//     28.0 / 29.2, 96 (12M) 41.2 / 33.9, 128 (16M) 43.6 / 36.6; 24 after 16000
+//     (12M) 44.5 / 33.3;
+//   32/4 heads of 64: 64 after 4000 (8M) 17.6 / 21.3, 96 (12M) 24.7 / 23.5,
+//     128 (16M) 26.1 / 25.7; 24 after 16000 (12M) 27.0 / 26.4;
+//   28/4 heads of 128: 64 after 4000 (7M) 28.2 / 29.6, 128 (14M) 43.1 / 34.6.
+// So from 11M rows x keys on it serves wherever it was measured faster, and
+// from 16384 rows on, where the grid is half full without a split, from 8M.
+// Below either line both kernels occur as the faster one: the 16-row kernels
+// lose where their groups have just begun another round, without context
+// from some 9000 rows on (32/8 heads of 128: 256 queries alone 18.3 / 18.7,
+// 320 32.4 / 23.9, 511 42.0 / 29.6, 512 41.9 / 29.4; of 64: 9.9 / 12.2, 18.8 /
+// 16.0, 24.8 / 18.6, 24.5 / 18.5; 28/4: 17.5 / 18.2, 31.9 / 22.8, 41.7 / 28.2,
+// 41.6 / 28.1), with fewer KV heads later (16/2: 511 22.0 / 24.3, 640 37.8 /
+// 26.3) and with context between (256 after 512 keys, 6M, 32/8 heads of 128
+// 25.7 / 27.6, after 1000, 10M, 48.5 / 31.9): these lines give that up.
 bool window_serves(int L_max, int nkv, int R) {
   const int64_t rows = (int64_t)nkv * R;
   return R >= 96 && rows * L_max >= (rows >= 16384 ? (int64_t)8 << 20 : (int64_t)11 << 20);
