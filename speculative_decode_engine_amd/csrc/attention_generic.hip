@@ -119,7 +119,7 @@ __device__ __forceinline__ void tile_load_to_lds(const char* p, uint32_t lds_off
       "global_load_lds_dwordx4 %1, off"
       :
       : "s"(lds_off), "v"(p)
-      : "memory", "m0");
+      : "memory");
 }
 
 // Byte offset of unit u of token t in a staged tile of U units per token:
