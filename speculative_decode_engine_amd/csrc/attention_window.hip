@@ -80,7 +80,7 @@ __device__ __forceinline__ void load_to_lds(const char* base, uint32_t off, uint
       "global_load_lds_dwordx4 %1, %2"
       :
       : "s"(lds_off), "v"(off), "s"(base)
-      : "memory", "m0");
+      : "memory");
 }
 
 // Waits for the wave's loads in flight.
