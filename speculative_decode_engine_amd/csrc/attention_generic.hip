@@ -111,7 +111,9 @@ struct TileLds {
 };
 
 // 16 bytes per lane from p into LDS at lds_off + 16 * lane (lds_off
-// wave-uniform); asynchronous (vmcnt).
+// wave-uniform); asynchronous (vmcnt).  m0 is a reserved register, which a
+// clobber list may not name: nothing else in the kernel may need it (nothing
+// does in the assembly of these kernels; LDS operations take no m0 here).
 __device__ __forceinline__ void tile_load_to_lds(const char* p, uint32_t lds_off) {
   asm volatile(
       "s_mov_b32 m0, %0\n\t"

@@ -72,7 +72,9 @@ struct WinShape {
 
 // 16 bytes per lane from base + off straight into LDS: lane l's go to
 // lds_off + 16l (lds_off wave-uniform).  Asynchronous (vmcnt); the memory
-// clobber and the waits below order it.
+// clobber and the waits below order it.  m0 is a reserved register, which a
+// clobber list may not name: nothing else in the kernel may need it (nothing
+// does in its assembly; LDS operations take no m0 here).
 __device__ __forceinline__ void load_to_lds(const char* base, uint32_t off, uint32_t lds_off) {
   asm volatile(
       "s_mov_b32 m0, %0\n\t"
