@@ -1,8 +1,11 @@
 // Paged GQA attention for any head_dim up to 512 and any block size, as
-// device code: the body of libsde_paged's generic kernel (the shapes its
-// MFMA tile kernels -- head_dim 64 / 128, block sizes that are multiples of
-// 8 -- do not take), and the block- and grid-cooperative forms the device
-// API (sde/attention_device.hpp) falls back to for those shapes.
+// device code: the fp32 work unit of the shapes that the MFMA tile kernels
+// (head_dim 64 / 128, block sizes that are multiples of 8) do not take.  In
+// libsde_paged it is the whole kernel for head sizes that are no multiple of 8
+// or above 256, and the others' matrix-core form (attention_generic.hip) runs
+// it where that form's sums are not finite; it is also the block- and
+// grid-cooperative form the device API (sde/attention_device.hpp) falls back
+// to for all of those shapes.
 //
 // Reference: device_flash_attention_gqa (attention.h:21-126) loops over any
 // dph.  This path keeps that generality with plain fp32 arithmetic: q fp32

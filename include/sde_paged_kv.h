@@ -190,18 +190,27 @@ size_t sde_grid_attention_workspace_size(int nh, int nkv, int dph, int n_queries
  * keys/values at positions [0, pos_base+m+1) of `layer`; query head h reads
  * KV head h*nkv/nh (attention.h:37); scale dph^-1/2.  n_queries = 1 is a
  * decode step, n_queries = k+1 the speculative verify window.
- * d_workspace may be NULL (the cache then keeps its own, grown on demand);
- * otherwise it must hold sde_paged_attention_workspace_size(...) bytes.
+ * d_workspace may be NULL (the cache then keeps its own, grown on demand by
+ * the first call that needs it, except under stream capture, where a call
+ * runs on what earlier calls made it: one that ran before, eagerly, captures;
+ * a split one that is the first gets SDE_ERR_WORKSPACE); otherwise it must
+ * hold sde_paged_attention_workspace_size(...) bytes.
  * Any dph up to 512 and any block size, nkv | nh, 1 <= n_queries <= 4096
  * (SDE_ERR_UNSUPPORTED for dph > 512): dph 64 / 128 with block sizes that
  * are multiples of 8 run the matrix-core tile kernels (those also need
- * nkv * ceil(n_queries * nh/nkv / 4) <= 4096), every other shape a plain
- * fp32 kernel with the same semantics and workspace.  The tile kernels
- * feed q * log2(e)/sqrt(dph) to the matrix cores as fp16 hi + lo parts, so
- * its elements must stay below 65504 in magnitude (|q| < 5.1e5 at dph 128,
- * 3.6e5 at dph 64; larger values overflow to Inf); the softmax weights are
- * at most 1.  Calls on one cache must be ordered on one stream (they share
- * the cache's arrival counters). */
+ * nkv * ceil(n_queries * nh/nkv / 4) <= 4096) or, for windows of many
+ * queries, the wide-window kernel; every other shape of a dph that is a
+ * multiple of 8 up to 256 a second matrix-core form, the rest a plain fp32
+ * kernel, all with the same semantics and the same workspace query.  The
+ * tile and wide-window kernels feed q * log2(e)/sqrt(dph) to the matrix cores
+ * as fp16 hi + lo parts, so its elements must stay below 65504 in magnitude
+ * (|q| < 5.1e5 at dph 128, 3.6e5 at dph 64; larger values overflow to Inf);
+ * their softmax weights, as fp16 pairs too, are at most 1 in the tile kernels
+ * and 2^15 in the wide-window kernel, whose quantum beside the largest is so
+ * much finer.  The second matrix-core form scales each row of q and the
+ * weights by powers of two (any finite q; its rows whose sums are not finite
+ * are done in fp32).  Calls on one cache must be ordered on one stream (they
+ * share the cache's arrival counters). */
 int sde_paged_attention(sde_kv_cache* cache, int layer, const float* d_q,
                         float* d_out, int nh, int nkv, int dph, int pos_base,
                         int n_queries, void* d_workspace,
@@ -210,9 +219,9 @@ int sde_paged_attention(sde_kv_cache* cache, int layer, const float* d_q,
 /* Bytes of the static device array sde_paged_attention_noalloc keeps its
  * partials in (one per device).  The tile kernels' partials (head sizes
  * 64 / 128) are at most (CUs x 16 rows) x (dph + 2) x 4 bytes, 2.1 MB on
- * MI355X's 256 CUs; the plain fp32 kernel of the other head sizes caps its
- * partition count so that its partials fit this size.  So on MI355X every
- * plan fits, and both entry points run the same plan. */
+ * MI355X's 256 CUs; the forms of the other shapes cap their partition count
+ * so that their partials fit this size.  So on MI355X every plan fits, and
+ * both entry points run the same plan. */
 #define SDE_NOALLOC_SCRATCH_BYTES ((size_t)4 << 20)
 
 /* Bytes of a second such array, for windows of many queries (a prompt or a
@@ -225,16 +234,17 @@ int sde_paged_attention(sde_kv_cache* cache, int layer, const float* d_q,
 #define SDE_NOALLOC_WIDE_SCRATCH_BYTES ((size_t)18 << 20)
 
 /* sde_paged_attention without a workspace, allocating nothing: the
- * split-context partials go to a static device array of the library
- * (SDE_NOALLOC_SCRATCH_BYTES per device, held until the process ends) and
+ * split-context partials go to static device arrays of the library
+ * (SDE_NOALLOC_SCRATCH_BYTES and, for wide windows,
+ * SDE_NOALLOC_WIDE_SCRATCH_BYTES per device, held until the process ends) and
  * the arrival counters are the cache's.  No counterpart in the reference:
  * it is for callers that cannot allocate device memory during the call --
  * code under HIP graph capture, tight serving loops, harnesses that forbid
  * allocation.  Same arguments, results and errors as sde_paged_attention
  * (minus the workspace), plus SDE_ERR_WORKSPACE for a call whose partials
- * would exceed the array.  The first call on a device looks up the array's
+ * would exceed its array.  The first call on a device looks up the array's
  * address there (with the cache's device current).  Every call on one GPU
- * shares that GPU's array: calls that overlap on one GPU (on different
+ * shares that GPU's arrays: calls that overlap on one GPU (on different
  * streams, or on different caches used concurrently) race on it and must
  * be ordered by the caller. */
 int sde_paged_attention_noalloc(sde_kv_cache* cache, int layer, const float* d_q,

@@ -58,9 +58,9 @@ __global__ __launch_bounds__(kThreads) void gen_rope_append_kernel(GenArgs a, Ge
 //  * the waves' sums meet in LDS, the partitions' in a combine kernel.
 // Bound by the latency of a few tiles in turn and, as they grow, by memory.
 // Measured on MI355X, us per layer, fp32 form / this: decode over 3000 keys,
-// 32 KV heads of 96, 188 + 13 (combine) / 17.3 in all; a 5-query window over
-// 4000 keys, 16/8 heads of 256, RoPE and the append included, 212 / 26.  Errors
-// against float64 fell too (4.7e-7 -> 3.0e-7, 6.5e-7 -> 4.2e-7 of the
+// 32 KV heads of 96, 188 + 13 (combine) / 14.4 + 3.8; a 5-query window over
+// 4000 keys, 16/8 heads of 256, RoPE and the append included, 212 / 26.5.
+// Errors against float64 fell too (4.7e-7 -> 2.4e-7, 6.4e-7 -> 3.4e-7 of the
 // output's norm): shorter sums.
 // DPHP: the head size rounded up to a multiple of 32.
 constexpr int kTileWaves = 4;

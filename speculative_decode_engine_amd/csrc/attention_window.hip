@@ -4,7 +4,7 @@
 // paged_attention.hip (query m of the window sees positions
 // [0, pos_base + m]; positions a row does not see never enter its sums).
 //
-// What bounds it is arithmetic: every K/V byte serves all rows of the window
+// What it costs is arithmetic: every K/V byte serves all rows of the window
 // and stays in the caches.  So, against the decode kernels' 16 rows per
 // workgroup with the waves splitting the context:
 //  * a workgroup holds 128 rows of one KV head, 32 per wave, and its waves
@@ -27,10 +27,13 @@
 // away on a fragmented pool, were waited for.
 //
 // Measured on MI355X: 2003 queries of 32/8 heads of 128, no context, 417 us
-// on the 16-row kernel (L2-bound: 4.1 GB read at ~10 TB/s), 98 here (33
-// GFLOP of products, twice that with the hi/lo split: 0.67 PFLOP/s of MFMA
-// work); 256 queries of 32/4 heads of 64 after 1500 keys 32.7 us, 20.7 + 4.1
-// for the combine here, of which ~5 us pass before the first tile arrives.
+// on the 16-row kernel (L2-bound: 4.1 GB read at ~10 TB/s), 97 here (33
+// GFLOP of products, twice that with the hi/lo split); 256 queries of 32/4
+// heads of 64 after 1500 keys 32.7 us, 20.7 + 4.6 for the combine here, of
+// which ~5 us pass before the first tile arrives.  Neither unit is full: of
+// the SIMD cycles of the long prompt the matrix cores are busy for 28 % and
+// the vector unit for 31 %, of the chunk's 13 % and 29 %; the waves wait a
+// third of their cycles for tiles and barriers and a third to issue.
 #include <hip/hip_runtime.h>
 
 #include "attention_window.hpp"
