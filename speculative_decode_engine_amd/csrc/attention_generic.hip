@@ -626,7 +626,7 @@ __global__ __launch_bounds__(kThreads) void gen_tile_combine_kernel(GenArgs a) {
     float4 x[8];
 #pragma unroll
     for (int k = 0; k < 8; k++) {
-      const int p = min(p0 + 4 * k, P - 1);  // (past the last: weight 0)
+      const int p = min(p0 + 4 * k, P - 1);
       ml[k] = mls[p];
       x[k] = *reinterpret_cast<const float4*>(acc + (int64_t)p * a.dph);
     }
@@ -642,7 +642,8 @@ __global__ __launch_bounds__(kThreads) void gen_tile_combine_kernel(GenArgs a) {
     o.w *= old;
 #pragma unroll
     for (int k = 0; k < 8; k++) {
-      const float w = p0 + 4 * k < P ? part_weight(ml[k], mx) : 0.f;
+      if (p0 + 4 * k >= P) break;  // (a weight of 0 would make NaN of Inf)
+      const float w = part_weight(ml[k], mx);
       l += ml[k].y * w;
       o.x += x[k].x * w;
       o.y += x[k].y * w;

@@ -118,6 +118,7 @@ def test_nonfinite_values_that_rows_see(gpu, oracle, nh, nkv, dph, bs, ctx, M, w
     if what == "V":
         V[7, ::3], V[90, 1::3] = np.inf, -np.inf
         V[40, dph - 1] = np.nan
+        V[ctx - 1, 5] = np.inf  # (in the last partition)
     elif what == "K":
         K[70, 3] = np.inf
         q.reshape(M, nh, dph)[:, ::2, 3] = -1.0
