@@ -598,7 +598,8 @@ __global__ __launch_bounds__(256) void window_combine_kernel(AttnArgs a) {
   float mx = -INFINITY, l = 0.f;
   float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
   // Batches of four partitions, every load of a batch in flight together
-  // (partitions past the last re-read it with weight 0).
+  // (partitions past the last re-read it and are left out: a weight of 0 would
+  // make NaN of Inf).
   for (int p0 = 0; p0 < P; p0 += 4) {
     float2 v[4];
     float4 x[4];
@@ -620,12 +621,13 @@ __global__ __launch_bounds__(256) void window_combine_kernel(AttnArgs a) {
     o.w *= old;
 #pragma unroll
     for (int i = 0; i < 4; i++) {
-      const float w = p0 + i >= P ? 0.f : sums_weight(v[i].x, v[i].y, mx);
-      l += v[i].y * w;
-      o.x += x[i].x * w;
-      o.y += x[i].y * w;
-      o.z += x[i].z * w;
-      o.w += x[i].w * w;
+      const bool in = p0 + i < P;
+      const float w = sums_weight(v[i].x, v[i].y, mx);
+      l += in ? v[i].y * w : 0.f;
+      o.x += in ? x[i].x * w : 0.f;
+      o.y += in ? x[i].y * w : 0.f;
+      o.z += in ? x[i].z * w : 0.f;
+      o.w += in ? x[i].w * w : 0.f;
     }
   }
   const float inv = attn::finish_scale(l);

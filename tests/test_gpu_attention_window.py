@@ -126,6 +126,25 @@ def test_wide_window_hidden_nonfinite_rows(gpu, oracle, dph):
     cache.free()
 
 
+def test_wide_window_combine_keeps_inf(gpu):
+    """Inf in V that every row sees, in the last partition of the rows before
+    position 4032 (576 tokens each): a part of a pair makes NaN of it where the
+    lo part is negative, as in every fp16 pair product here, but the combine of
+    seven partitions must not."""
+    case_banner("wide window, Inf in the last partition")
+    nh, nkv, dph, bs, ctx, M = 32, 8, 128, 16, 4000, 128
+    cache, K, V, rng = build_layer(nh, nkv, dph, bs, ctx, M, 270, 3)
+    v = V[3900:3901].copy()
+    v[0, 7] = np.inf
+    cache.append(0, torch.from_numpy(K[3900:3901].copy()).cuda(), torch.from_numpy(v).cuda(), 3900)
+    q = torch.from_numpy(W.queries(rng, M, nh, dph)).cuda()
+    out = cache.attention(0, q, nh, nkv, dph, ctx).view(M, nh, dph)
+    assert not torch.isfinite(out[:, :4, 7]).any()
+    assert torch.isfinite(out[:, :, 8:]).all() and torch.isfinite(out[:, 4:]).all()
+    assert (out[:32, :4, 7] == float("inf")).any() and (out[32:, :4, 7] == float("inf")).any()
+    cache.free()
+
+
 def test_wide_window_replays_in_a_graph(gpu):
     """Captured with a workspace, and captured with none on a cache that owns
     none yet (one partition then): replays match the eager call."""
